@@ -14,6 +14,7 @@
 #include <thread>
 #include <vector>
 
+#include "hsdc_fold.h"
 #include "hsdc_internal.h"
 #include "hsdc_hss.h"
 #include "hsdc_hss_host.h"
@@ -1195,9 +1196,9 @@ static int run_merges(hsdc_ctx *c, const Merge *dm, const std::vector<Merge> &hm
                            c->dlvlmax + SEC_SLOTS * std::min(c->cur_level, SEC_LEVELS - 1));
         prof_mark(c, -1);
         prof_mark(c, 1);
-        hipLaunchKernelGGL(k_loewner, dim3(chunkK[nm]), dim3(WGS), 0, s, dmg, dchunkK, nm, dmo, W);
+        hipLaunchKernelGGL(k_loewner, dim3(fold_grid(chunkK[nm])), dim3(OF_WG), 0, s, dmg, dchunkK, nm, dmo, W);
         prof_mark(c, -1);
-        hipLaunchKernelGGL(k_sbuild, dim3(chunkK[nm]), dim3(WGS), 0, s, dmg, dchunkK, nm, dmo, dsoff, W,
+        hipLaunchKernelGGL(k_sbuild, dim3(fold_grid(chunkK[nm])), dim3(OF_WG), 0, s, dmg, dchunkK, nm, dmo, dsoff, W,
                            (double *)c->sb.p);
         if (!tiles.empty())
             hipLaunchKernelGGL(k_gemm, dim3(tiles.size()), dim3(WGS), 0, s, dmg, dtiles, (int)tiles.size(),
@@ -1211,7 +1212,7 @@ static int run_merges(hsdc_ctx *c, const Merge *dm, const std::vector<Merge> &hm
             if (!ho[i].flags && ho[i].hss && ho[i].k > 0) sel.push_back(i);
         if (!sel.empty()) {  // after k_newcols: the products go into the slots it assigned
             prof_mark(c, 1);
-            hipLaunchKernelGGL(k_alpha, dim3(chunkK[nm]), dim3(WGS), 0, s, dmg, dchunkK, nm, dmo, W);
+            hipLaunchKernelGGL(k_alpha, dim3(fold_grid(chunkK[nm])), dim3(OF_WG), 0, s, dmg, dchunkK, nm, dmo, W);
             prof_mark(c, -1);
             CK(run_hss(c, dmg, hm, m0, ho, sel, dprobs, cur, gbase));
         }
@@ -1308,10 +1309,10 @@ static int level_dev(hsdc_ctx *c, const Merge *dmg, const std::vector<Merge> &hm
                        c->dlvlmax + SEC_SLOTS * std::min(L, SEC_LEVELS - 1));
     prof_mark(c, -1);
     prof_mark(c, 1);
-    hipLaunchKernelGGL(k_loewner, dim3(totN), dim3(WGS), 0, s, dmg, (const int *)t.chunkK, nm,
+    hipLaunchKernelGGL(k_loewner, dim3(fold_grid(totN)), dim3(OF_WG), 0, s, dmg, (const int *)t.chunkK, nm,
                        (const MergeOut *)dmo, W);
     prof_mark(c, -1);
-    hipLaunchKernelGGL(k_sbuild, dim3(totN), dim3(WGS), 0, s, dmg, (const int *)t.chunkK, nm, (const MergeOut *)dmo,
+    hipLaunchKernelGGL(k_sbuild, dim3(fold_grid(totN)), dim3(OF_WG), 0, s, dmg, (const int *)t.chunkK, nm, (const MergeOut *)dmo,
                        (const long *)t.soff, W, (double *)c->sb.p);
     if (B.tiles > 0)
         hipLaunchKernelGGL(k_gemm, dim3(dev_grid(B.tiles)), dim3(WGS), 0, s, dmg, (const GTile *)nullptr, 0,
@@ -1349,7 +1350,7 @@ static int level_hss(hsdc_ctx *c, const Merge *dmg, const std::vector<Merge> &hm
     if (sel.empty()) return 0;
     Work W = c->W;
     prof_mark(c, 1);
-    hipLaunchKernelGGL(k_alpha, dim3(totN), dim3(WGS), 0, s, dmg, (const int *)t.chunkK, nm, (const MergeOut *)dmo,
+    hipLaunchKernelGGL(k_alpha, dim3(fold_grid(totN)), dim3(OF_WG), 0, s, dmg, (const int *)t.chunkK, nm, (const MergeOut *)dmo,
                        W);
     prof_mark(c, -1);
     CK(run_hss(c, dmg, hm, 0, ho, sel, dprobs, cur, gbase));  // writes the new vectors into their slots
@@ -2383,9 +2384,9 @@ int hsdc_laed3(hsdc_ctx *c, int k, int n, int n1, double *d, double *q, int ldq,
                            1, (const MergeOut *)dmo, W, c->dsec);
     hipLaunchKernelGGL(k_secular, dim3(tabs[1]), dim3(SEC_WG), 0, s, (const Merge *)dm, (const int *)dtab, 1,
                        (const MergeOut *)dmo, W, c->prm.maxit, dinfo, c->dsec, c->dlvlmax);
-    hipLaunchKernelGGL(k_loewner, dim3(tabs[3]), dim3(WGS), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
+    hipLaunchKernelGGL(k_loewner, dim3(fold_grid(tabs[3])), dim3(OF_WG), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
                        (const MergeOut *)dmo, W);
-    hipLaunchKernelGGL(k_sbuild, dim3(tabs[3]), dim3(WGS), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
+    hipLaunchKernelGGL(k_sbuild, dim3(fold_grid(tabs[3])), dim3(OF_WG), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
                        (const MergeOut *)dmo, (const long *)c->lvl.p, W, (double *)c->sb.p);
     // the two GEMMs of DLAED3 with the packed Q2 (types 1,2 rows on top, 2,3 below)
     const double *S = (const double *)c->sb.p, *Q2 = (const double *)c->xb.p;
@@ -2438,9 +2439,9 @@ int hsdc_loewner(hsdc_ctx *c, int k, double rho, double *dlamda, double *z, doub
                            1, (const MergeOut *)dmo, W, c->dsec);
     hipLaunchKernelGGL(k_secular, dim3(tabs[1]), dim3(SEC_WG), 0, s, (const Merge *)dm, (const int *)dtab, 1,
                        (const MergeOut *)dmo, W, c->prm.maxit, dinfo, c->dsec, c->dlvlmax);
-    hipLaunchKernelGGL(k_loewner, dim3(tabs[3]), dim3(WGS), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
+    hipLaunchKernelGGL(k_loewner, dim3(fold_grid(tabs[3])), dim3(OF_WG), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
                        (const MergeOut *)dmo, W);
-    hipLaunchKernelGGL(k_alpha, dim3(tabs[3]), dim3(WGS), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
+    hipLaunchKernelGGL(k_alpha, dim3(fold_grid(tabs[3])), dim3(OF_WG), 0, s, (const Merge *)dm, (const int *)(dtab + 2), 1,
                        (const MergeOut *)dmo, W);
     HK(hipGetLastError());
     int info = 0;

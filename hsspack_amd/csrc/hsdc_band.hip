@@ -29,6 +29,7 @@
 #include <mutex>
 #include <vector>
 
+#include "hsdc_fold.h"
 #include "hsdc_internal.h"
 #include "hsdc_hss.h"
 #include "../../include/hsdc.h"
@@ -1147,12 +1148,12 @@ int sb_solve(hsdc_sb_ctx *c, int lower, int n, int kd, const double *dab, long l
                                up, kd);
             hipLaunchKernelGGL(k_secular, dim3(gsec), dim3(SEC_WG), 0, st, (const Merge *)dm2, (const int *)T.secblk,
                                nm, (const MergeOut *)dmo, W, c->prm.maxit, dinfo, dsec, dlvm);
-            hipLaunchKernelGGL(k_loewner, dim3(gch), dim3(BWG), 0, st, (const Merge *)dm2, (const int *)T.chunk, nm,
+            hipLaunchKernelGGL(k_loewner, dim3(fold_grid(gch)), dim3(OF_WG), 0, st, (const Merge *)dm2, (const int *)T.chunk, nm,
                                (const MergeOut *)dmo, W);
             if (!hsel.empty())
-                hipLaunchKernelGGL(k_alpha, dim3(gch), dim3(BWG), 0, st, (const Merge *)dm2, (const int *)T.chunk,
+                hipLaunchKernelGGL(k_alpha, dim3(fold_grid(gch)), dim3(OF_WG), 0, st, (const Merge *)dm2, (const int *)T.chunk,
                                    nm, (const MergeOut *)dmo, W);
-            hipLaunchKernelGGL(k_sbuild, dim3(gch), dim3(BWG), 0, st, (const Merge *)dm2, (const int *)T.chunk, nm,
+            hipLaunchKernelGGL(k_sbuild, dim3(fold_grid(gch)), dim3(OF_WG), 0, st, (const Merge *)dm2, (const int *)T.chunk, nm,
                                (const MergeOut *)dmo, so, W, (double *)c->s.p);
             if (L.nmax >= 4096)  // wide tiles where they fill the chip (same bits as k_bgemm)
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bgemm_w<256, 128, 16, 1, 2, 4>),

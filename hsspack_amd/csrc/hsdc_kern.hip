@@ -10,6 +10,7 @@
 // returns bit-identical roots, index sets and rotations.
 #include <climits>
 #include <cmath>
+#include "hsdc_fold.h"
 #include "hsdc_internal.h"
 #include "hsdc_mlp.h"
 
@@ -1363,195 +1364,217 @@ __device__ __forceinline__ double delta_ij(const double *d, int i, const int *or
 // Loewner z of the dense branch, LAPACK DLAED3 order: W(I) = DELTA_I(I) times
 // DELTA_I(J)/(DLAMDA(I)-DLAMDA(J)) for J ascending, z = sign(sqrt(-W), w).
 // Also the HSS branch (MDLAED3, mdlaed3.f90:207-230): product from 1 with the
-// J = I factor taken in place, z = sign(sqrt|prod|, w).  One thread per I; the
-// poles, tau and origins of a merge with K <= LW_LDS are staged in LDS first
-// (every thread walks all K of them).
-#define LW_LDS 2048
-#define LW_U 8
-__global__ __launch_bounds__(WG) void k_loewner(const Merge *mg, const int *chunk_start, int nm,
-                                                const MergeOut *mo, Work W)
+// J = I factor taken in place, z = sign(sqrt|prod|, w).  An ordered fold of one
+// quotient per pole (hsdc_fold.h); the divide's operands are selected, not its
+// result (1.0 / 1.0 and num / 1.0 are exact).
+struct LoewnerTerm {
+    struct Raw { double d; int o; double t; };
+    const double *d, *tau;
+    const int *org;
+    double di;
+    int i;
+    bool hss;
+    __device__ __forceinline__ Raw raw(int p) const { return Raw{d[p], org[p], tau[p]}; }
+    __device__ __forceinline__ void vals(const Raw &r, double *v) const { v[0] = r.d; v[1] = d[r.o - 1]; v[2] = r.t; }
+    // delta_i(j) = (d_i - d_org(j)) - tau_j, as delta_ij forms it
+    template <int W>
+    __device__ __forceinline__ double term(const double *v, int p) const
+    {
+        const bool self = W == 0 && p == i;
+        const double num = (di - v[OF_P]) - v[2 * OF_P], den = di - v[0];
+        return ((self && !hss) ? 1.0 : num) / (self ? 1.0 : den);
+    }
+    __device__ __forceinline__ double fold(double a, double t) const { return a * t; }
+};
+
+template <int R>
+__device__ __forceinline__ void loewner_block(const MergeOut &o, int s, int r0, Work &W, FoldLds<3> &S)
+{
+    const int K = o.k, lane = threadIdx.x & 63, i = r0 + (lane & (R - 1));
+    LoewnerTerm f{W.dlamda + s, W.tau + s, W.org + s, 0.0, i, o.hss != 0};
+    const int ic = min(i, K - 1);
+    f.di = f.d[ic];
+    double wv = (threadIdx.x >= 512 && !o.hss) ? delta_ij(f.d, ic, f.org, f.tau, ic) : 1.0;
+    wv = ordered_fold<R>(f, K, r0, wv, S);
+    if (threadIdx.x >= 512 && lane < R && i < K)
+        W.wnew[s + i] = o.hss ? copysign(sqrt(fabs(wv)), W.w[s + i]) : copysign(sqrt(-wv), W.w[s + i]);
+}
+
+__global__ __launch_bounds__(OF_WG) void k_loewner(const Merge *mg, const int *chunk_start, int nm,
+                                                   const MergeOut *mo, Work W)
 {
     if (gate_closed(W, mg)) return;
-    // chunks of LW_LDS poles: d_j, d_org(j) and tau_j staged by the block, every
-    // thread's product walks them in order
-    __shared__ double sd[LW_LDS], so[LW_LDS], st[LW_LDS];
-    const int nvb = chunk_start[nm];
-    for (int vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
-        const int m = find_seg(chunk_start, nm, vb);
+    __shared__ FoldLds<3> S;
+    const int nch = chunk_start[nm];
+    const FoldSplit P = fold_split(nch);
+    for (int vb = blockIdx.x; vb < nch * P.parts; vb += gridDim.x) {
+        const int ch = vb / P.parts, m = find_seg(chunk_start, nm, ch);
         const MergeOut o = mo[m];
+        const int c0 = (ch - chunk_start[m]) * 256, r0 = c0 + (vb % P.parts) * P.R;
         if (o.flags || o.k < 3) continue;  // uniform over the block
-        const int s = mg[m].s, K = o.k, i = (vb - chunk_start[m]) * WG + threadIdx.x;
-        const double *d = W.dlamda + s, *tau = W.tau + s;
-        const int *org = W.org + s;
-        const bool own = i < K;
-        const double di = own ? d[i] : 0.0;
-        // delta_i(j) = (d_i - d_org(j)) - tau_j, as delta_ij forms it
-        double wv = (own && !o.hss) ? delta_ij(d, i, org, tau, i) : 1.0;
-        for (int c0 = 0; c0 < K; c0 += LW_LDS) {
-            const int cn = min(LW_LDS, K - c0);
-            for (int t = threadIdx.x; t < cn; t += WG) {
-                sd[t] = d[c0 + t];
-                so[t] = d[org[c0 + t] - 1];
-                st[t] = tau[c0 + t];
-            }
-            __syncthreads();
-            if (own) {
-                // factor of pole J: the quotient, or at J = I nothing (dense: times 1.0,
-                // which leaves the product's bits as they are) or the numerator (HSS).
-                // LW_U quotients are formed independently, then multiplied into the
-                // product in J order: a level launches one thread per root, too few
-                // wavefronts to hide the divide and LDS latency of one pole at a time.
-                // The divide's operands are selected, not its result (1.0 / 1.0 and
-                // num / 1.0 are exact), so every pole runs the same straight-line code.
-                const int me = i - c0;
-                const bool hss = o.hss;
-                int jj = 0;
-                for (; jj + LW_U <= cn; jj += LW_U) {
-                    double f[LW_U];
-#pragma unroll
-                    for (int u = 0; u < LW_U; u++) {
-                        const bool self = jj + u == me;
-                        const double num = (di - so[jj + u]) - st[jj + u], den = di - sd[jj + u];
-                        f[u] = ((self && !hss) ? 1.0 : num) / (self ? 1.0 : den);
-                    }
-#pragma unroll
-                    for (int u = 0; u < LW_U; u++) wv = wv * f[u];
-                }
-                for (; jj < cn; jj++) {
-                    const bool self = jj == me;
-                    const double num = (di - so[jj]) - st[jj], den = di - sd[jj];
-                    wv = wv * (((self && !hss) ? 1.0 : num) / (self ? 1.0 : den));
-                }
-            }
-            __syncthreads();  // the next chunk or virtual block restages
+        const int s = mg[m].s, end = min(o.k, c0 + 256);
+        for (int r = r0; r < end; r += P.parts * P.R) {
+            if (P.R == 64) loewner_block<64>(o, s, r, W, S);
+            else loewner_block<16>(o, s, r, W, S);
         }
-        if (own) W.wnew[s + i] = o.hss ? copysign(sqrt(fabs(wv)), W.w[s + i]) : copysign(sqrt(-wv), W.w[s + i]);
     }
 }
 
 // Dense branch eigenvector matrix of the secular problem (DLAED3, after label
 // 70): S(t,j) = (W(I)/DELTA_I(J)) / ||W./DELTA(:,J)||, I = INDXC(t); written
-// row-major (S[t*K + j]) so one lane per column stores coalesced.  Poles, Loewner
-// z and INDXC of a merge with K <= LW_LDS are staged in LDS.
-__global__ __launch_bounds__(WG) void k_sbuild(const Merge *mg, const int *chunk_start, int nm,
-                                               const MergeOut *mo, const long *soff, Work W, double *S)
+// row-major (S[t*K + j]).  The squares of a column are an ordered fold (the sum runs
+// over i in order); then the block spreads the column's K entries over its threads,
+// with the poles and the Loewner z of a merge with K <= SB_LDS staged in INDXC order
+// in the fold's buffer.  With a thread per column for the sum (K dependent divides at
+// about 125 ns each) a level of two merges of K = 1400 took 182 us.
+struct NormTerm {
+    struct Raw { double d, w; };
+    const double *d, *wz;
+    double dorg, tj;
+    __device__ __forceinline__ Raw raw(int p) const { return Raw{d[p], wz[p]}; }
+    __device__ __forceinline__ void vals(const Raw &r, double *v) const { v[0] = r.d; v[1] = r.w; }
+    // delta_i(j) = (d_i - d_org(j)) - tau_j, as delta_ij forms it
+    template <int W>
+    __device__ __forceinline__ double term(const double *v, int) const
+    {
+        const double q = v[OF_P] / ((v[0] - dorg) - tj);
+        return q * q;
+    }
+    __device__ __forceinline__ double fold(double a, double t) const { return a + t; }
+};
+#define SB_LDS 4096  // 2 x SB_LDS doubles fit the fold's buffer
+
+template <int R>
+__device__ __forceinline__ void sbuild_block(int K, int s, int c0, const Work &W, double *Sm, FoldLds<2> &L,
+                                             double *nrm)
+{
+    const double *d = W.dlamda + s, *wz = W.wnew + s;
+    const int *indxc = W.indxc + s;
+    const int tid = threadIdx.x, jl = tid & (R - 1), j = c0 + jl, jc = min(j, K - 1);
+    NormTerm f{d, wz, 0.0, W.tau[s + jc]};
+    f.dorg = d[W.org[s + jc] - 1];
+    const double acc = ordered_fold<R>(f, K, c0, 0.0, L);
+    if (tid >= 512 && (tid & 63) < R) nrm[tid & 63] = sqrt(acc);
+    const bool stg = K <= SB_LDS;
+    double *sd = &L.buf[0][0], *sw = sd + SB_LDS;
+    if (stg)
+        for (int t = tid; t < K; t += OF_WG) {
+            const int i = indxc[t] - 1;
+            sd[t] = d[i];
+            sw[t] = wz[i];
+        }
+    __syncthreads();
+    const double temp = nrm[jl];
+    if (j < K) {
+        constexpr int RPP = OF_WG / R;  // rows per pass
+#pragma unroll 4
+        for (int t = tid / R; t < K; t += RPP) {
+            double dv, wv;
+            if (stg) {
+                dv = sd[t];
+                wv = sw[t];
+            } else {
+                const int i = indxc[t] - 1;
+                dv = d[i];
+                wv = wz[i];
+            }
+            Sm[(long)t * K + j] = (wv / ((dv - f.dorg) - f.tj)) / temp;
+        }
+    }
+    __syncthreads();  // the next virtual block restages
+}
+
+__global__ __launch_bounds__(OF_WG) void k_sbuild(const Merge *mg, const int *chunk_start, int nm,
+                                                  const MergeOut *mo, const long *soff, Work W, double *S)
 {
     if (gate_closed(W, mg)) return;
-    __shared__ double sd[LW_LDS], sw[LW_LDS];
-    __shared__ int sc[LW_LDS];
-    __shared__ double sdo[WG], stj[WG], stm[WG];  // per column of the block: d_org, tau, norm
-    const int nvb = chunk_start[nm];
-    for (int vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
-        const int m = find_seg(chunk_start, nm, vb);
+    __shared__ FoldLds<2> L;
+    __shared__ double nrm[64];
+    const int nch = chunk_start[nm];
+    const FoldSplit P = fold_split(nch);
+    for (int vb = blockIdx.x; vb < nch * P.parts; vb += gridDim.x) {
+        const int ch = vb / P.parts, m = find_seg(chunk_start, nm, ch);
         const MergeOut o = mo[m];
-        if (o.flags || o.hss || o.k == 0) continue;  // uniform over the block
-        const int s = mg[m].s, K = o.k, j = (vb - chunk_start[m]) * WG + threadIdx.x;
+        const int c0 = (ch - chunk_start[m]) * 256, r0 = c0 + (vb % P.parts) * P.R, K = o.k;
+        if (o.flags || o.hss || r0 >= K) continue;  // uniform over the block
+        const int s = mg[m].s, end = min(K, c0 + 256);
         double *Sm = S + soff[m];
-        const int *indxc = W.indxc + s;
         if (K <= 2) {
+            const int j = threadIdx.x;
             if (j < K) {
                 if (K == 1) {
                     Sm[0] = 1.0;
                 } else {
                     double dv[2] = {W.difl[s + j], W.difr[s + j]};
-                    for (int t = 0; t < 2; t++) Sm[t * K + j] = dv[indxc[t] - 1];
+                    for (int t = 0; t < 2; t++) Sm[t * K + j] = dv[W.indxc[s + t] - 1];
                 }
             }
             continue;
         }
-        const double *d = W.dlamda + s, *wz = W.wnew + s;
-        if (K <= LW_LDS) {
-            for (int t = threadIdx.x; t < K; t += WG) { sd[t] = d[t]; sw[t] = wz[t]; sc[t] = indxc[t]; }
-            __syncthreads();
-            d = sd; wz = sw; indxc = sc;
+        for (int r = r0; r < end; r += P.parts * P.R) {
+            if (P.R == 64) sbuild_block<64>(K, s, r, W, Sm, L, nrm);
+            else sbuild_block<16>(K, s, r, W, Sm, L, nrm);
         }
-        // column norms, one thread per column j (the sum runs over i in order);
-        // delta_i(j) = (d_i - d_org(j)) - tau_j, as delta_ij forms it
-        if (j < K) {
-            const double dorg = d[W.org[s + j] - 1], tj = W.tau[s + j];
-            double acc = 0.0;
-            for (int i = 0; i < K; i++) {
-                double v = wz[i] / ((d[i] - dorg) - tj);
-                acc += v * v;
-            }
-            sdo[threadIdx.x] = dorg;
-            stj[threadIdx.x] = tj;
-            stm[threadIdx.x] = sqrt(acc);
-        }
-        __syncthreads();
-        // the K x ncols entries, spread over all threads: WG / ncols rows per pass
-        const int c0 = j - threadIdx.x, ncols = min(WG, K - c0), rpp = WG / ncols;
-        const int jj = threadIdx.x % ncols, t0 = threadIdx.x / ncols;
-        if (t0 < rpp) {
-            const double dorg = sdo[jj], tj = stj[jj], temp = stm[jj];
-            for (int t = t0; t < K; t += rpp) {
-                int i = indxc[t] - 1;
-                Sm[(long)t * K + c0 + jj] = (wz[i] / ((d[i] - dorg) - tj)) / temp;
-            }
-        }
-        __syncthreads();  // the next virtual block restages
     }
 }
 
-// HSS branch scalars (mdlaed3.f90:215-249): DIFL, DIFR, alpha_j = 1/||col j||.
-// One thread per column j; the poles and Loewner z are staged in chunks of LW_LDS.
-__global__ __launch_bounds__(WG) void k_alpha(const Merge *mg, const int *chunk_start, int nm,
-                                              const MergeOut *mo, Work W)
+// HSS branch scalars (mdlaed3.f90:215-249): DIFL, DIFR, alpha_j = 1/||col j||, the
+// squares of a column an ordered fold.  Entry i = j: wz_j / difl; i < j and i > j: the
+// differences from lambda_j's two neighbouring poles.
+struct AlphaTerm {
+    struct Raw { double d, w; };
+    const double *d, *wz;
+    double difl, difrj, dlamj, dlamjp;
+    int j;
+    __device__ __forceinline__ Raw raw(int p) const { return Raw{d[p], wz[p]}; }
+    __device__ __forceinline__ void vals(const Raw &r, double *v) const { v[0] = r.d; v[1] = r.w; }
+    template <int W>
+    __device__ __forceinline__ double term(const double *v, int i) const
+    {
+        const double dlo = (v[0] + dlamj) - difl, dhi = (v[0] + dlamjp) + difrj;
+        const double q = v[OF_P] / (W == 1 ? dlo : W == 2 ? dhi : (i == j) ? difl : (i < j) ? dlo : dhi);
+        return q * q;
+    }
+    __device__ __forceinline__ double fold(double a, double t) const { return a + t; }
+};
+
+template <int R>
+__device__ __forceinline__ void alpha_block(int K, int s, int r0, Work &W, FoldLds<2> &S)
+{
+    const double *d = W.dlamda + s, *tau = W.tau + s, *wz = W.wnew + s;
+    const int *org = W.org + s;
+    const int lane = threadIdx.x & 63, j = r0 + (lane & (R - 1)), jc = min(j, K - 1);
+    const bool own = threadIdx.x >= 512 && lane < R && j < K;
+    AlphaTerm f{d, wz, 0.0, 0.0, 0.0, 0.0, j};
+    f.difl = -delta_ij(d, jc, org, tau, jc);
+    const double difr = (jc + 1 < K) ? -delta_ij(d, jc + 1, org, tau, jc) : 0.0;
+    f.dlamj = -d[jc];
+    if (jc + 1 < K) { f.difrj = -difr; f.dlamjp = -d[jc + 1]; }
+    if (own) {
+        W.difl[s + j] = f.difl;
+        W.difr[s + j] = difr;
+    }
+    const double acc = ordered_fold<R>(f, K, r0, 0.0, S);
+    if (own) W.alpha[s + j] = 1.0 / sqrt(acc);
+}
+
+__global__ __launch_bounds__(OF_WG) void k_alpha(const Merge *mg, const int *chunk_start, int nm,
+                                                 const MergeOut *mo, Work W)
 {
     if (gate_closed(W, mg)) return;
-    __shared__ double sd[LW_LDS], sw[LW_LDS];
-    const int nvb = chunk_start[nm];
-    for (int vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
-        const int m = find_seg(chunk_start, nm, vb);
+    __shared__ FoldLds<2> S;
+    const int nch = chunk_start[nm];
+    const FoldSplit P = fold_split(nch);
+    for (int vb = blockIdx.x; vb < nch * P.parts; vb += gridDim.x) {
+        const int ch = vb / P.parts, m = find_seg(chunk_start, nm, ch);
         const MergeOut o = mo[m];
+        const int c0 = (ch - chunk_start[m]) * 256, r0 = c0 + (vb % P.parts) * P.R;
         if (o.flags || !o.hss) continue;  // uniform over the block
-        const int s = mg[m].s, K = o.k, j = (vb - chunk_start[m]) * WG + threadIdx.x;
-        const double *d = W.dlamda + s, *tau = W.tau + s, *wz = W.wnew + s;
-        const int *org = W.org + s;
-        const bool own = j < K;
-        double difl = 0.0, difr = 0.0, dlamj = 0.0, difrj = 0.0, dlamjp = 0.0, wzj = 0.0;
-        if (own) {
-            difl = -delta_ij(d, j, org, tau, j);
-            difr = (j + 1 < K) ? -delta_ij(d, j + 1, org, tau, j) : 0.0;
-            W.difl[s + j] = difl;
-            W.difr[s + j] = difr;
-            dlamj = -d[j];
-            if (j + 1 < K) { difrj = -difr; dlamjp = -d[j + 1]; }
-            wzj = wz[j];
+        const int s = mg[m].s, end = min(o.k, c0 + 256);
+        for (int r = r0; r < end; r += P.parts * P.R) {
+            if (P.R == 64) alpha_block<64>(o.k, s, r, W, S);
+            else alpha_block<16>(o.k, s, r, W, S);
         }
-        double acc = 0.0;
-        for (int c0 = 0; c0 < K; c0 += LW_LDS) {
-            const int cn = min(LW_LDS, K - c0);
-            for (int t = threadIdx.x; t < cn; t += WG) { sd[t] = d[c0 + t]; sw[t] = wz[c0 + t]; }
-            __syncthreads();
-            // column entry i = j: wz_j / difl; i < j and i > j: the differences from
-            // lambda_j's two neighbouring poles.  LW_U entries are formed
-            // independently, then summed in i order (one thread per column, so few
-            // wavefronts per level that one entry at a time leaves the latency bare).
-            if (own) {
-                int ii = 0;
-                for (; ii + LW_U <= cn; ii += LW_U) {
-                    double v[LW_U];
-#pragma unroll
-                    for (int u = 0; u < LW_U; u++) {
-                        const int i = c0 + ii + u;
-                        const double dlo = (sd[ii + u] + dlamj) - difl, dhi = (sd[ii + u] + dlamjp) + difrj;
-                        v[u] = ((i == j) ? wzj : sw[ii + u]) / ((i == j) ? difl : (i < j) ? dlo : dhi);
-                    }
-#pragma unroll
-                    for (int u = 0; u < LW_U; u++) acc += v[u] * v[u];
-                }
-                for (; ii < cn; ii++) {
-                    const int i = c0 + ii;
-                    const double den = (i == j) ? difl
-                                     : (i < j) ? (sd[ii] + dlamj) - difl : (sd[ii] + dlamjp) + difrj;
-                    const double v = ((i == j) ? wzj : sw[ii]) / den;
-                    acc += v * v;
-                }
-            }
-            __syncthreads();  // the next chunk or virtual block restages
-        }
-        if (own) W.alpha[s + j] = 1.0 / sqrt(acc);
     }
 }
 

@@ -7,6 +7,7 @@
 #include <stddef.h>
 #include <string.h>
 
+#include "hsdc_fold.h"
 #include "hsdc_internal.h"
 #include "../../include/hsdc.h"
 
@@ -133,8 +134,8 @@ extern "C" int hsdc_loewner_noalloc(int k, double rho, const double *d_dlamda, c
     hipLaunchKernelGGL(k_na_setup, dim3(1), dim3(256), 0, s, b, k, rho, d_info);
     hipLaunchKernelGGL(k_secular, dim3(nsec), dim3(SEC_WG), 0, s, dm, tab, 1, dmo, W, 100, d_info,
                        (const SecCtl *)(b + O_SEC), (unsigned int *)(b + O_LVL));
-    hipLaunchKernelGGL(k_loewner, dim3(nch), dim3(256), 0, s, dm, tab + 2, 1, dmo, W);
-    hipLaunchKernelGGL(k_alpha, dim3(nch), dim3(256), 0, s, dm, tab + 2, 1, dmo, W);
+    hipLaunchKernelGGL(k_loewner, dim3(fold_grid(nch)), dim3(OF_WG), 0, s, dm, tab + 2, 1, dmo, W);
+    hipLaunchKernelGGL(k_alpha, dim3(fold_grid(nch)), dim3(OF_WG), 0, s, dm, tab + 2, 1, dmo, W);
     if (hipGetLastError() != hipSuccess) return HSDC_ERR_HIP;
     return 0;
 }

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "../../include/hsdc.h"
+#include "hsdc_fold.h"
 #include "hsdc_internal.h"
 #include "hsdc_hss.h"
 
@@ -970,63 +971,59 @@ __global__ __launch_bounds__(256) void k_bd_secular(const BdMerge *mg, int nmg, 
 }
 
 // ------------------------------------------------------------------------------
-// updated z (DLASD3, Loewner form): thread per index, products in DLASD3's order.
-// DLASD3's two loops (J < I with pole D(J), J >= I with D(J+1)) are one product over
-// J = 1 .. K-1 ascending; each lane picks the pole by its own I.  The block stages
-// chunks of (D(ORG(J)), TAU(J), D(J)) in LDS and forms BL_U factors at a time before
-// multiplying them in order: a level launches one thread per index, too few
-// wavefronts to hide the latency of one factor at a time.
+// updated z (DLASD3, Loewner form), products in DLASD3's order.  DLASD3's two loops
+// (J < I with pole D(J), J >= I with D(J+1)) are one product over J = 1 .. K-1
+// ascending, each index picking the pole by its own I: an ordered fold of one term
+// (two divides) per J (hsdc_fold.h).
 // ------------------------------------------------------------------------------
-#define BL_LDS 2048
-#define BL_U 8
-__global__ __launch_bounds__(256) void k_bd_loewner(const BdMerge *mg, int nmg, BdTab tab, BdWork W, const BdOut *mo)
+struct BdLoewnerTerm {
+    struct Raw { int o; double t, d0, d1; };
+    const double *ds, *tau;
+    const int *org;
+    double di;
+    int i;  // 1-based
+    __device__ __forceinline__ Raw raw(int p) const { return Raw{org[p], tau[p], ds[p], ds[p + 1]}; }
+    __device__ __forceinline__ void vals(const Raw &r, double *v) const
+    {
+        v[0] = ds[r.o - 1]; v[1] = r.t; v[2] = r.d0; v[3] = r.d1;
+    }
+    // J = p + 1: pole D(J) below I, D(J+1) from I on
+    template <int W>
+    __device__ __forceinline__ double term(const double *v, int p) const
+    {
+        const double dd = W == 1 || (W == 0 && p + 1 < i) ? v[2 * OF_P] : v[3 * OF_P];
+        return sv_den(di, v[0], v[OF_P]) / (di - dd) / (di + dd);
+    }
+    __device__ __forceinline__ double fold(double a, double t) const { return a * t; }
+};
+
+template <int R>
+__device__ __forceinline__ void bd_loewner_block(int k, int s, int r0, const BdWork &W, FoldLds<4> &S)
 {
-  __shared__ double so[BL_LDS], st[BL_LDS], sdd[BL_LDS + 1];
-  const int tot = tab.low[nmg];
-  for (int b = blockIdx.x; b < tot; b += gridDim.x) {
-    const int mi = bd_find(tab.low, nmg, b);  // uniform over the block
-    const int s = mg[mi].s, k = mo[mi].k;
-    const int i = (b - tab.low[mi]) * 256 + threadIdx.x + 1;  // 1-based
-    const bool own = i <= k;
-    const double *ds = W.dsg + s;
-    const double di = own ? ds[i - 1] : 0.0;
-    double zi = own ? sv_den(di, ds[W.org[s + k - 1] - 1], W.tau[s + k - 1]) : 1.0;
-    for (int c0 = 1; c0 <= k - 1; c0 += BL_LDS) {
-      const int cn = min(BL_LDS, k - c0);  // J = c0 .. c0 + cn - 1
-      for (int t = threadIdx.x; t < cn; t += 256) {
-        const int j = c0 + t;
-        so[t] = ds[W.org[s + j - 1] - 1];
-        st[t] = W.tau[s + j - 1];
-        sdd[t] = ds[j - 1];
-      }
-      if (threadIdx.x == 0) sdd[cn] = ds[c0 + cn - 1];
-      __syncthreads();
-      if (own) {
-        // pole of J: D(J) = sdd[t] below I, D(J+1) = sdd[t + 1] from I on
-        const int sw = i - c0;  // first t with J >= I
-        int t = 0;
-        for (; t + BL_U <= cn; t += BL_U) {
-          double f[BL_U];
-#pragma unroll
-          for (int u = 0; u < BL_U; u++) {
-            const double dd = (t + u < sw) ? sdd[t + u] : sdd[t + u + 1];
-            f[u] = sv_den(di, so[t + u], st[t + u]) / (di - dd) / (di + dd);
-          }
-#pragma unroll
-          for (int u = 0; u < BL_U; u++) zi = zi * f[u];
-        }
-        for (; t < cn; t++) {
-          const double dd = (t < sw) ? sdd[t] : sdd[t + 1];
-          zi = zi * (sv_den(di, so[t], st[t]) / (di - dd) / (di + dd));
-        }
-      }
-      __syncthreads();  // the next chunk or block restages
+    const int lane = threadIdx.x & 63, i = r0 + (lane & (R - 1)) + 1, ic = min(i, k);
+    BdLoewnerTerm f{W.dsg + s, W.tau + s, W.org + s, 0.0, i};
+    f.di = f.ds[ic - 1];
+    double zi = sv_den(f.di, f.ds[f.org[k - 1] - 1], f.tau[k - 1]);
+    zi = ordered_fold<R>(f, k - 1, r0, zi, S);
+    if (threadIdx.x >= 512 && lane < R && i <= k) {
+        const double a = sqrt(fabs(zi));
+        W.zl[s + i - 1] = W.zs[s + i - 1] >= 0.0 ? a : -a;
     }
-    if (own) {
-      const double a = sqrt(fabs(zi));
-      W.zl[s + i - 1] = W.zs[s + i - 1] >= 0.0 ? a : -a;
+}
+
+__global__ __launch_bounds__(OF_WG) void k_bd_loewner(const BdMerge *mg, int nmg, BdTab tab, BdWork W, const BdOut *mo)
+{
+    __shared__ FoldLds<4> S;
+    const int nch = tab.low[nmg];
+    const FoldSplit P = fold_split(nch);
+    for (int vb = blockIdx.x; vb < nch * P.parts; vb += gridDim.x) {
+        const int ch = vb / P.parts, mi = bd_find(tab.low, nmg, ch);  // uniform over the block
+        const int s = mg[mi].s, k = mo[mi].k, c0 = (ch - tab.low[mi]) * 256, end = min(k, c0 + 256);
+        for (int r = c0 + (vb % P.parts) * P.R; r < end; r += P.parts * P.R) {
+            if (P.R == 64) bd_loewner_block<64>(k, s, r, W, S);
+            else bd_loewner_block<16>(k, s, r, W, S);
+        }
     }
-  }
 }
 
 // ------------------------------------------------------------------------------
@@ -2024,7 +2021,7 @@ static int bd_solve(hsdc_bd_ctx *c, int n, const std::vector<double> &he, double
         hipLaunchKernelGGL(k_bd_znorm, dim3(nm), dim3(64), 0, st, mg, W, mo);
         hipLaunchKernelGGL(k_bd_secular, dim3(g_sec[t]), dim3(256), 0, st, mg, nm, tab, W, (const BdOut *)mo,
                            c->prm.maxit, dfail);
-        hipLaunchKernelGGL(k_bd_loewner, dim3(g_low[t]), dim3(256), 0, st, mg, nm, tab, W, (const BdOut *)mo);
+        hipLaunchKernelGGL(k_bd_loewner, dim3(fold_grid(g_low[t])), dim3(OF_WG), 0, st, mg, nm, tab, W, (const BdOut *)mo);
         hipLaunchKernelGGL(k_bd_vec, dim3(g_sec[t]), dim3(256), 0, st, mg, nm, tab, W, (const BdOut *)mo, Q);
         hipLaunchKernelGGL(k_bd_gemm, dim3(g_tile[t]), dim3(256), 0, st, mg, nm, tab, W, (const BdOut *)mo,
                            (const double *)Q, (const double *)U, (const double *)V, ld, S);
