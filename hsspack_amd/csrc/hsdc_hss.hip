@@ -144,30 +144,69 @@ __device__ VI block_argmax(VI x, VI *sh)
     return r;
 }
 
-// The same with one barrier: successive calls alternate between the two halves of sh
-// (4 x blockDim / 64 entries; a half holds 2 x blockDim / 64 so that the two-value
+// v of the lane CTRL names, or v itself where that lane is outside the row
+template <int CTRL>
+__device__ __forceinline__ double dpp_max(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)(unsigned)b, hi = (int)(b >> 32);
+    const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
+    const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
+    return fmax(v, __longlong_as_double(((long long)h2 << 32) | (unsigned)l2));
+}
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(unsigned)b, l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// The (value, smallest index) maximum over the wavefront's first NL lanes (64 or 8), in
+// every lane, for values >= 0: the values go through a prefix of DPP moves (no LDS
+// traffic), the index is read from the lane a ballot finds.  A butterfly of (value,
+// index) pairs, three of whose six steps cross lanes through LDS, took about 1000 cycles
+// for two reductions; this takes about 300.
+template <int NL>
+__device__ __forceinline__ VI wave_argmax(VI x)
+{
+    const double v = x.i > 0 ? x.v : -1.0;
+    double m = dpp_max<0x111>(v);  // row_shr:1
+    m = dpp_max<0x112>(m);
+    m = dpp_max<0x114>(m);
+    if (NL == 64) {
+        m = dpp_max<0x118>(m);
+        m = dpp_max<0x142>(m);  // row_bcast:15
+        m = dpp_max<0x143>(m);  // row_bcast:31
+    }
+    m = lane_value(m, NL - 1);
+    constexpr unsigned long long LN = NL == 64 ? ~0ull : (1ull << (NL & 63)) - 1;
+    unsigned long long b = __ballot(x.i > 0 && v == m) & LN;
+    if (b == 0) b = __ballot(x.i > 0) & LN;  // no number among the values
+    if (b == 0) return VI{0.0, 0};
+    int l = __builtin_ctzll(b);
+    int i = __builtin_amdgcn_readlane(x.i, l);
+    for (b &= b - 1; b; b &= b - 1) {
+        const int l2 = __builtin_ctzll(b), i2 = __builtin_amdgcn_readlane(x.i, l2);
+        if (i2 < i) { i = i2; l = l2; }
+    }
+    return VI{lane_value(x.v, l), i};
+}
+// Over the block with one barrier: successive calls alternate between the two halves of
+// sh (4 x blockDim / 64 entries; a half holds 2 x blockDim / 64 so that the two-value
 // form below shares them), so a call's writes never meet the previous call's reads
 // and the trailing barrier that protects a single buffer is not needed.  tog is
-// uniform over the block and flips on every call.
-// With wave set the block is one wavefront: every lane holds the maximum after the
-// butterfly, and nothing goes through sh.
+// uniform over the block and flips on every call.  Blocks of 4 or 8 wavefronts.
+// With wave set the block is one wavefront, and nothing goes through sh.
 __device__ __forceinline__ VI block_argmax_t(VI x, VI *sh, int &tog, bool wave = false)
 {
     const int tid = threadIdx.x, nw = (int)(blockDim.x >> 6);
     VI *b = sh + tog * 2 * nw;
     tog ^= 1;
-    x = vi_step<32>(x);
-    x = vi_step<16>(x);
-    x = vi_step<8>(x);
-    x = vi_step<4>(x);
-    x = vi_step<2>(x);
-    x = vi_step<1>(x);
+    x = wave_argmax<64>(x);
     if (wave) return x;
     if ((tid & 63) == 0) b[tid >> 6] = x;
     __syncthreads();
-    VI r = b[0];
-    for (int w = 1; w < nw; w++) r = vi_better(r, b[w]);
-    return r;
+    return wave_argmax<8>(b[tid & (nw - 1)]);
 }
 // Two independent (value, index) maxima under one barrier, in the same alternating
 // halves of sh.
@@ -176,19 +215,32 @@ __device__ __forceinline__ void block_argmax2_t(VI &x, VI &y, VI *sh, int &tog, 
     const int tid = threadIdx.x, nw = (int)(blockDim.x >> 6);
     VI *b = sh + tog * 2 * nw;
     tog ^= 1;
-    x = vi_step<32>(x); y = vi_step<32>(y);
-    x = vi_step<16>(x); y = vi_step<16>(y);
-    x = vi_step<8>(x); y = vi_step<8>(y);
-    x = vi_step<4>(x); y = vi_step<4>(y);
-    x = vi_step<2>(x); y = vi_step<2>(y);
-    x = vi_step<1>(x); y = vi_step<1>(y);
+    x = wave_argmax<64>(x);
+    y = wave_argmax<64>(y);
     if (wave) return;
     if ((tid & 63) == 0) { b[tid >> 6] = x; b[nw + (tid >> 6)] = y; }
     __syncthreads();
-    VI rx = b[0], ry = b[nw];
-    for (int w = 1; w < nw; w++) { rx = vi_better(rx, b[w]); ry = vi_better(ry, b[nw + w]); }
-    x = rx;
-    y = ry;
+    x = wave_argmax<8>(b[tid & (nw - 1)]);
+    y = wave_argmax<8>(b[nw + (tid & (nw - 1))]);
+}
+// lanes per column of the swap check's scan: the k columns' rows are spread over all NTH
+// threads, G (a power of two) to a column
+__device__ __forceinline__ int scan_lanes(int k, int NTH)
+{
+    int g = 1;
+    while (g < 64 && 2 * g * k <= NTH) g *= 2;
+    return g;
+}
+// (value, smallest index) maximum over aligned groups of g lanes
+__device__ __forceinline__ VI group_argmax(VI x, int g)
+{
+    if (g > 32) x = vi_step<32>(x);
+    if (g > 16) x = vi_step<16>(x);
+    if (g > 8) x = vi_step<8>(x);
+    if (g > 4) x = vi_step<4>(x);
+    if (g > 2) x = vi_step<2>(x);
+    if (g > 1) x = vi_step<1>(x);
+    return x;
 }
 // The block's barrier, or for a one-wavefront block the ordering of its LDS accesses
 // (a wavefront executes in lockstep; the fence completes lane 0's writes before any
@@ -281,7 +333,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
     int tog = 0;  // which half of red the next reduction uses
     __shared__ long s_off;
     __shared__ int s_M, s_N, s_Rk, s_flag, s_ii, s_jj;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     constexpr int RB = HSS_CWG >= 512 ? (SQ ? 6 : 7) : 4;  // within 256 VGPRs
     if ((int)blockIdx.x >= nn) return;
     HssNode Nd = nodes[blockIdx.x];
@@ -355,19 +407,35 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
             if (SQ) Rl[4 * NS + j] = r.s;
         }
     }
-    // column swap (one thread; a barrier follows)
+    // column swap (one thread; a barrier follows): every load before the first store, so
+    // that their latencies overlap
     auto swapc = [&](int a, int c) {
-        double t = vld(a); vst(a, vld(c)); vst(c, t);
-        int u = pu(a), w = pu(c);
+        const double va = vld(a), vc = vld(c);
+        const int u = pu(a), w = pu(c);
+        double ra[RD], rc[RD];
+        if (sm) {
+            #pragma unroll
+            for (int q = 0; q < RD; q++) { ra[q] = Rl[q * NS + a - 1]; rc[q] = Rl[q * NS + c - 1]; }
+        }
+        vst(a, vc); vst(c, va);
         pu_set(a, w); pu_set(c, u);
         if (a <= mn) A1(PUs, a) = w;
         if (c <= mn) A1(PUs, c) = u;
         if (sm) {
             #pragma unroll
-            for (int q = 0; q < RD; q++) {
-                t = Rl[q * NS + a - 1]; Rl[q * NS + a - 1] = Rl[q * NS + c - 1]; Rl[q * NS + c - 1] = t;
-            }
+            for (int q = 0; q < RD; q++) { Rl[q * NS + a - 1] = rc[q]; Rl[q * NS + c - 1] = ra[q]; }
         }
+    };
+    // row swap of the generators, likewise
+    auto swapr = [&](int a, int c) {
+        const double fa = A1(F, a), fc = A1(F, c), za = A1(Z, a), zc = A1(Z, c), aa = A1(A, a), ac = A1(A, c);
+        const int la = A1(PL, a), lc2 = A1(PL, c);
+        const short qa = A1(PQ, a), qc = A1(PQ, c);
+        A1(F, a) = fc; A1(F, c) = fa;
+        A1(Z, a) = zc; A1(Z, c) = za;
+        A1(A, a) = ac; A1(A, c) = aa;
+        A1(PL, a) = lc2; A1(PL, c) = la;
+        A1(PQ, a) = qc; A1(PQ, c) = qa;
     };
     auto cload = [&](int j0, int *pw, double *v) {
         #pragma unroll
@@ -387,8 +455,21 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
     auto cpass = [&](int lo, auto body) {
         int j0 = lo + tid;
         if (j0 > N) return;
-        if (sm) {
-            for (int j = j0; j <= N; j += NTH) body(j, A1(PUl, j), A1(Vl, j), rl_get(j));
+        if (sm) {  // two columns at a time: their LDS loads and divides overlap
+            for (int j = j0; j <= N; j += 2 * NTH) {
+                const int p0 = A1(PUl, j);
+                const double v0 = A1(Vl, j);
+                const RootG c0r = rl_get(j);
+                if (j - lane + NTH <= N) {  // uniform over the wavefront
+                    const int j1 = min(j + NTH, N), p1 = A1(PUl, j1);
+                    const double v1 = A1(Vl, j1);
+                    const RootG c1r = rl_get(j1);
+                    body(j, p0, v0, c0r);
+                    body(j + NTH, p1, v1, c1r);
+                } else {
+                    body(j, p0, v0, c0r);
+                }
+            }
             return;
         }
         int pw[RB];
@@ -424,6 +505,14 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         for (int i = k + tid; i <= M; i += NTH)
             x = vi_better(x, VI{fabs(A1(Z, i) / fd_r<SQ>(A1(F, i), A1(PL, i), pw, w)), i - k + 1});
         return x;
+    };
+    // the same over the block's rows on every wavefront by itself: for few rows a second
+    // or third pass over them costs less than a reduction over the block
+    auto rowsearch_w = [&](int k, int pw, const RootG &w) -> VI {
+        VI x = {0.0, 0};
+        for (int i = k + lane; i <= M; i += 64)
+            x = vi_better(x, VI{fabs(A1(Z, i) / fd_r<SQ>(A1(F, i), A1(PL, i), pw, w)), i - k + 1});
+        return wave_argmax<64>(x);
     };
     for (int i = tid; i < M; i += NTH) {
         PL[i] = A1((gcint *)H.PL, l0 + i);
@@ -466,24 +555,16 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
             if (!(junkL <= piv && junkU <= piv)) {
                 int flg = (junkL > junkU) ? 1 : 0;
                 int jjL = cl.i, jjU = rw.i;
-                // Every thread has read position k for the tests above before any swap.
-                // A row swap is made after the column search it feeds, which reads the
-                // incoming row where it still is; every later swap follows a reduction,
-                // whose barrier comes after all reads of the previous search.
-                bsync(wave);
+                // Every thread has read position k for the tests above before any swap: a
+                // row swap is made after the column search it feeds (which reads the
+                // incoming row where it still is) and its reduction's barrier.
+                if (flg == 0) bsync(wave);
                 for (;;) {
                     if (flg == 1) {
                         const int jr = jjL + k - 1;
                         jjU = block_argmax_t(colsearch(k, A1(PL, jr), A1(F, jr)), red, tog, wave).i;
                         fl += 4ull * (N - k + 1);
-                        if (tid == 0) {
-                            double t;
-                            t = A1(F, k); A1(F, k) = A1(F, jr); A1(F, jr) = t;
-                            t = A1(Z, k); A1(Z, k) = A1(Z, jr); A1(Z, jr) = t;
-                            t = A1(A, k); A1(A, k) = A1(A, jr); A1(A, jr) = t;
-                            int u = A1(PL, k); A1(PL, k) = A1(PL, jr); A1(PL, jr) = u;
-                            short q = A1(PQ, k); A1(PQ, k) = A1(PQ, jr); A1(PQ, jr) = q;
-                        }
+                        if (tid == 0) swapr(k, jr);
                         if (jjU == 1) {
                             bsync(wave);
                             break;
@@ -493,15 +574,19 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                     bsync(wave);
                     const int pwk2 = A1(PUs, k);
                     cw = croot(k);
-                    jjL = block_argmax_t(rowsearch(k, pwk2, cw), red, tog, wave).i;
+                    const bool few = M - k < 256;
+                    jjL = few ? rowsearch_w(k, pwk2, cw).i : block_argmax_t(rowsearch(k, pwk2, cw), red, tog, wave).i;
                     fl += 4ull * (M - k + 1);
-                    if (jjL == 1) break;
+                    if (jjL == 1) {
+                        if (few) bsync(wave);  // before the update pass writes what the search reads
+                        break;
+                    }
                     flg = 1;
                 }
             }
         }
-        // every swap of the search is followed by a barrier and the search only reads, so
-        // the update pass below may start without another
+        // the search ended with a barrier after its last swap and its last reads (or made
+        // none), so the update pass below may start without another
         double ukk = A1(Z, k) * vld(k) / fd_r<SQ>(A1(F, k), A1(PL, k), A1(PUs, k), cw);
         amax = fmax(amax, fabs(ukk));
         if (fabs(ukk) < tol * amax) {
@@ -545,14 +630,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
             bsync(wave);
             if (tid == 0) {
                 int ii = s_ii, jj = s_jj;
-                int a = ii + k - 1, b = jj + k - 1;
-                double t;
-                t = A1(F, k); A1(F, k) = A1(F, a); A1(F, a) = t;
-                t = A1(Z, k); A1(Z, k) = A1(Z, a); A1(Z, a) = t;
-                t = A1(A, k); A1(A, k) = A1(A, a); A1(A, a) = t;
-                int u = A1(PL, k); A1(PL, k) = A1(PL, a); A1(PL, a) = u;
-                short q = A1(PQ, k); A1(PQ, k) = A1(PQ, a); A1(PQ, a) = q;
-                swapc(k, b);
+                swapr(k, ii + k - 1);
+                swapc(k, jj + k - 1);
             }
             bsync(wave);
             cw = croot(k);
@@ -571,6 +650,20 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         const double ff1 = fuse ? A1(F, k + 1) : 0.0;
         const int pun = fuse ? A1(PUs, k + 1) : puk;
         const RootG cn = fuse ? croot(k + 1) : cw;
+        // The last wavefront updates W and forms W(k), an ordered product, while the others
+        // are in their passes: its factors' gathers in parallel, then lane 0 multiplies.
+        // W and T1 are touched by this wavefront alone until the barrier below.
+        if (tid >= NTH - 64) {
+            for (int j = k - 1 - lane; j >= 1; j -= 64) {
+                double temp = -1.0 * fd_r<SQ>(A1(F, j), A1(PL, j), puk, ck);
+                A1(W, j) = A1(W, j) * (temp / ppq<SQ>(Fk, A1(F, j)));
+                const int puj = A1(PUs, j);
+                const double t2 = -1.0 * fd_r<SQ>(Fk, plk, puj, croot(j));
+                A1(T1, j) = t2 / ppq<SQ>(A1(F, j), Fk);
+            }
+            bsync(true);
+            if (lane == 0) A1(W, k) = ordered_prod(fd_r<SQ>(Fk, plk, puk, ck) / A1(A, k), T1, k - 1);
+        }
         VI x1 = {0.0, 0};
         for (int j = k + 1 + tid; j <= M; j += NTH) {
             double temp = fd_r<SQ>(A1(F, j), A1(PL, j), puk, ck);
@@ -590,25 +683,9 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                 if (fuse) y1 = vi_better(y1, VI{fabs(vj / fd_r<SQ>(ff1, fk1, pw, c)), j - k});
             }
         });
-        // j = k - 1 on thread 0, which wrote W(k - 1) at the end of the previous step: a
-        // fused step has no barrier between that write and this loop.  For the same
-        // reason the factors of W(k) go to T1 and T2 on alternate steps (thread 0 may
-        // still read the previous step's; the swap check uses both only after a barrier)
-        double *Tk = (k & 1) ? T2 : T1;
-        for (int j = k - 1 - tid; j >= 1; j -= NTH) {
-            double temp = -1.0 * fd_r<SQ>(A1(F, j), A1(PL, j), puk, ck);
-            A1(W, j) = A1(W, j) * (temp / ppq<SQ>(Fk, A1(F, j)));
-            // the factors of W(k) (their gathers in parallel; the product stays in order)
-            const int puj = A1(PUs, j);
-            const double t2 = -1.0 * fd_r<SQ>(Fk, plk, puj, croot(j));
-            A1(Tk, j) = t2 / ppq<SQ>(A1(F, j), Fk);
-        }
         fl += 5ull * (M - k) + 7ull * (N - k) + 12ull * (k - 1);
         pre = fuse;
-        // The reduction's barrier also publishes the update pass (T1 for thread 0's
-        // product), and the next step reads W(k) only after its own first barrier, so a
-        // fused step needs no other; before a swap check, and at the last step, W(k) is
-        // published here.
+        // The reduction's barrier (or the one before a swap check) publishes the passes and W
         if (fuse) {
             block_argmax2_t(x1, y1, red, tog, wave);
             pre_cl = x1;
@@ -617,28 +694,26 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         } else {
             bsync(wave);
         }
-        if (tid == 0) {
-            double wk = fd_r<SQ>(Fk, plk, puk, ck) / A1(A, k);
-            wk = ordered_prod(wk, Tk, k - 1);
-            A1(W, k) = wk;
-        }
-        if (!fuse) bsync(wave);
         // ---- every 10 steps: swap while max |Mat_N| > rho (searchMax2Eig)
         if (k % 10 == 0 && M - k > 0) {
             for (;;) {
+                // per column the first largest entry over the rows, G lanes to a column (one
+                // thread per column took 30-60 thousand cycles a check)
                 VI x = {0.0, 0};
-                for (int jc = 1 + tid; jc <= k; jc += NTH) {
-                    double fj = A1(F, jc), mv = 0.0;
-                    int mi = 0;
-                    for (int i = 1; i <= M - k; i++) {
-                        double v = fabs(A1(Z, k + i) / ppq<SQ>(A1(F, k + i), fj));
-                        if (mi == 0 || v > mv) { mv = v; mi = i; }
+                const int G = scan_lanes(k, NTH), g = tid & (G - 1);
+                for (int jc = 1 + tid / G; jc - tid / G <= k; jc += NTH / G) {
+                    VI e = {0.0, 0};
+                    if (jc <= k) {
+                        const double fj = A1(F, jc);
+                        for (int i = 1 + g; i <= M - k; i += G)
+                            e = vi_better(e, VI{fabs(A1(Z, k + i) / ppq<SQ>(A1(F, k + i), fj)), i});
                     }
-                    double junk = mv * fabs(A1(W, jc));
-                    VI c = {junk, jc};
-                    VI nb = vi_better(x, c);
-                    if (nb.i == jc) IP[jc - 1] = (short)mi;
-                    x = nb;
+                    e = group_argmax(e, G);
+                    if (jc <= k) {
+                        const VI nb = vi_better(x, VI{e.v * fabs(A1(W, jc)), jc});
+                        if (nb.i == jc && g == 0) IP[jc - 1] = (short)e.i;
+                        x = nb;
+                    }
                 }
                 VI win = block_argmax_t(x, red, tog, wave);
                 if (!(win.v > rho)) break;
@@ -690,9 +765,9 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         }
     }
     // ---- U generator (CauchylikeEigQ, then rows back to the node order)
+    for (int i = 1 + tid; i <= M; i += NTH) IP[A1(PQ, i) - 1] = (short)i;  // invp
     if (tid == 0) {
         atomicAdd(H.flops, fl);
-        for (int i = 1; i <= M; i++) IP[A1(PQ, i) - 1] = i;  // invp
         int r = Rk;
         if (r < mn) {
             s_Rk = r;
@@ -756,7 +831,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
     int tog = 0;  // which half of red the next reduction uses
     __shared__ long s_off;
     __shared__ int s_M, s_N, s_Rk, s_flag, s_ii, s_jj;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     constexpr int RB = HSS_CWG >= 512 ? 8 : 4;
     if ((int)blockIdx.x >= nn) return;
     HssNode Nd = nodes[blockIdx.x];
@@ -826,20 +901,34 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
     }
     // outside-row swap (one thread; a barrier follows)
     auto swapc = [&](int a, int c) {
-        double t = vld(a); vst(a, vld(c)); vst(c, t);
-        int u = pu(a), w = pu(c);
+        const double va = vld(a), vc = vld(c);
+        const int u = pu(a), w = pu(c);
+        const double fa = sm ? A1(FFl, a) : 0.0, fc = sm ? A1(FFl, c) : 0.0;
+        vst(a, vc); vst(c, va);
         pu_set(a, w); pu_set(c, u);
         if (a <= mn) A1(PUs, a) = w;
         if (c <= mn) A1(PUs, c) = u;
-        if (sm) { t = A1(FFl, a); A1(FFl, a) = A1(FFl, c); A1(FFl, c) = t; }
+        if (sm) { A1(FFl, a) = fc; A1(FFl, c) = fa; }
     };
-    // node-column swap of the root values (one thread, beside the swaps of Dr, Z, A, PL, PQ)
-    auto swapr = [&](int a, int c) {
+    // node-column swap of Dr, A, PL, PQ and the root values; of Z too unless the swap check
+    // replaces Z (zs)
+    auto swapr = [&](int a, int c, bool zs) {
+        const double da = A1(Dr, a), dc = A1(Dr, c), za = A1(Z, a), zc = A1(Z, c), aa = A1(A, a), ac = A1(A, c);
+        const int la = A1(PL, a), lc2 = A1(PL, c);
+        const short qa = A1(PQ, a), qc = A1(PQ, c);
+        double ra[RD], rc[RD];
         if (sm) {
             #pragma unroll
-            for (int q = 0; q < RD; q++) {
-                double t = RRl[q * M + a - 1]; RRl[q * M + a - 1] = RRl[q * M + c - 1]; RRl[q * M + c - 1] = t;
-            }
+            for (int q = 0; q < RD; q++) { ra[q] = RRl[q * M + a - 1]; rc[q] = RRl[q * M + c - 1]; }
+        }
+        A1(Dr, a) = dc; A1(Dr, c) = da;
+        if (zs) { A1(Z, a) = zc; A1(Z, c) = za; }
+        A1(A, a) = ac; A1(A, c) = aa;
+        A1(PL, a) = lc2; A1(PL, c) = la;
+        A1(PQ, a) = qc; A1(PQ, c) = qa;
+        if (sm) {
+            #pragma unroll
+            for (int q = 0; q < RD; q++) { RRl[q * M + a - 1] = rc[q]; RRl[q * M + c - 1] = ra[q]; }
         }
     };
     auto cload = [&](int j0, int *pd, double *v) {
@@ -859,8 +948,19 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
     auto cpass = [&](int lo, auto body) {
         int j0 = lo + tid;
         if (j0 > N) return;
-        if (sm) {
-            for (int j = j0; j <= N; j += NTH) body(j, A1(PUl, j), A1(Vl, j), A1(FFl, j));
+        if (sm) {  // two rows at a time: their LDS loads and divides overlap
+            for (int j = j0; j <= N; j += 2 * NTH) {
+                const int p0 = A1(PUl, j);
+                const double v0 = A1(Vl, j), f0 = A1(FFl, j);
+                if (j - lane + NTH <= N) {  // uniform over the wavefront
+                    const int j1 = min(j + NTH, N), p1 = A1(PUl, j1);
+                    const double v1 = A1(Vl, j1), f1 = A1(FFl, j1);
+                    body(j, p0, v0, f0);
+                    body(j + NTH, p1, v1, f1);
+                } else {
+                    body(j, p0, v0, f0);
+                }
+            }
             return;
         }
         int pd[RB];
@@ -896,6 +996,13 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
         for (int i = k + tid; i <= M; i += NTH)
             x = vi_better(x, VI{fabs(A1(Z, i) / fd_r<SQ>(ffd, pd, A1(PL, i), rroot(i))), i - k + 1});
         return x;
+    };
+    // the same on every wavefront by itself, as in the row compression
+    auto rowsearch_w = [&](int k, int pd, double ffd) -> VI {
+        VI x = {0.0, 0};
+        for (int i = k + lane; i <= M; i += 64)
+            x = vi_better(x, VI{fabs(A1(Z, i) / fd_r<SQ>(ffd, pd, A1(PL, i), rroot(i))), i - k + 1});
+        return wave_argmax<64>(x);
     };
     for (int i = tid; i < M; i += NTH) {
         Dr[i] = A1((gdbl *)H.D, c0 + i);
@@ -953,9 +1060,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
             if (!(junkL <= piv && junkU <= piv)) {
                 int flg = (junkL > junkU) ? 1 : 0;
                 int jjL = cl.i, jjU = rw.i;
-                // barriers as in the row compression: one before the first swap, then a
-                // row swap after the column search it feeds
-                bsync(wave);
+                // barriers as in the row compression
+                if (flg == 0) bsync(wave);
                 for (;;) {
                     if (flg == 1) {
                         const int jr = jjL + k - 1;
@@ -963,15 +1069,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                         cr = rroot(jr);
                         jjU = block_argmax_t(colsearch(k, plr, cr), red, tog, wave).i;
                         fl += 4ull * (N - k + 1);
-                        if (tid == 0) {
-                            double t;
-                            t = A1(Dr, k); A1(Dr, k) = A1(Dr, jr); A1(Dr, jr) = t;
-                            t = A1(Z, k); A1(Z, k) = A1(Z, jr); A1(Z, jr) = t;
-                            t = A1(A, k); A1(A, k) = A1(A, jr); A1(A, jr) = t;
-                            int u = A1(PL, k); A1(PL, k) = A1(PL, jr); A1(PL, jr) = u;
-                            short q = A1(PQ, k); A1(PQ, k) = A1(PQ, jr); A1(PQ, jr) = q;
-                            swapr(k, jr);
-                        }
+                        if (tid == 0) swapr(k, jr, true);
                         if (jjU == 1) {
                             bsync(wave);
                             break;
@@ -981,15 +1079,18 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                     bsync(wave);
                     const int puk2 = A1(PUs, k);
                     ffp = A1(FF, puk2);
-                    jjL = block_argmax_t(rowsearch(k, puk2, ffp), red, tog, wave).i;
+                    const bool few = M - k < 256;
+                    jjL = few ? rowsearch_w(k, puk2, ffp).i : block_argmax_t(rowsearch(k, puk2, ffp), red, tog, wave).i;
                     fl += 4ull * (M - k + 1);
-                    if (jjL == 1) break;
+                    if (jjL == 1) {
+                        if (few) bsync(wave);  // before the update pass writes what the search reads
+                        break;
+                    }
                     flg = 1;
                 }
             }
         }
-        // every swap of the search is followed by a barrier and the search only reads, so
-        // the update pass below may start without another
+        // the search ended with a barrier, as in the row compression
         double ukk = A1(Z, k) * vld(k) / (-1.0 * fd_r<SQ>(ffp, A1(PUs, k), A1(PL, k), cr));
         amax = fmax(amax, fabs(ukk));
         if (fabs(ukk) < tol * amax) {
@@ -1030,15 +1131,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
             if (win.i > 0 && best.i == win.i) { s_ii = bestrow; s_jj = win.i; }
             bsync(wave);
             if (tid == 0) {
-                int a = s_ii + k - 1, b = s_jj + k - 1;
-                double t;
-                t = A1(Dr, k); A1(Dr, k) = A1(Dr, a); A1(Dr, a) = t;
-                t = A1(Z, k); A1(Z, k) = A1(Z, a); A1(Z, a) = t;
-                t = A1(A, k); A1(A, k) = A1(A, a); A1(A, a) = t;
-                int u = A1(PL, k); A1(PL, k) = A1(PL, a); A1(PL, a) = u;
-                short q = A1(PQ, k); A1(PQ, k) = A1(PQ, a); A1(PQ, a) = q;
-                swapr(k, a);
-                swapc(k, b);
+                swapr(k, s_ii + k - 1, true);
+                swapc(k, s_jj + k - 1);
             }
             bsync(wave);
             cr = rroot(k);
@@ -1055,6 +1149,22 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
         const int pun = fuse ? A1(PUs, k + 1) : puk;
         const RootG ck1 = fuse ? rroot(k + 1) : ck;
         const double ffn = A1(FF, pun);
+        // W on the last wavefront, as in the row compression
+        if (tid >= NTH - 64) {
+            for (int j = k - 1 - lane; j >= 1; j -= 64) {
+                const int plj = A1(PL, j), puj = A1(PUs, j);
+                const RootG rj = rroot(j);
+                double temp = fd_r<SQ>(Fk, puk, plj, rj);
+                double temp2 = dd_r<SQ>(plk, ck, plj, rj);
+                temp = temp / temp2;
+                A1(W, j) = A1(W, j) * temp;
+                temp = fd_r<SQ>(sm ? A1(FFl, j) : A1(FF, puj), puj, plk, ck);
+                temp2 = dd_r<SQ>(plj, rj, plk, ck);
+                A1(T1, j) = temp / temp2;
+            }
+            bsync(true);
+            if (lane == 0) A1(W, k) = ordered_prod((-1.0 * fd_r<SQ>(Fk, puk, plk, ck)) / A1(A, k), T1, k - 1);
+        }
         VI x1 = {0.0, 0};
         for (int j = k + 1 + tid; j <= M; j += NTH) {
             const int plj = A1(PL, j);
@@ -1075,24 +1185,9 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                 if (fuse) y1 = vi_better(y1, VI{fabs(vj / fd_r<SQ>(ffd, pd, plk1, ck1)), j - k});
             }
         });
-        // j = k - 1 on thread 0, and the factors of W(k) in T1 or T2 by the step's
-        // parity, as in the row compression
-        double *Tk = (k & 1) ? T2 : T1;
-        for (int j = k - 1 - tid; j >= 1; j -= NTH) {
-            const int plj = A1(PL, j), puj = A1(PUs, j);
-            const RootG rj = rroot(j);
-            double temp = fd_r<SQ>(Fk, puk, plj, rj);
-            double temp2 = dd_r<SQ>(plk, ck, plj, rj);
-            temp = temp / temp2;
-            A1(W, j) = A1(W, j) * temp;
-            // the factors of W(k) (their gathers in parallel; the product stays in order)
-            temp = fd_r<SQ>(sm ? A1(FFl, j) : A1(FF, puj), puj, plk, ck);
-            temp2 = dd_r<SQ>(plj, rj, plk, ck);
-            A1(Tk, j) = temp / temp2;
-        }
         fl += 6ull * (M - k) + 5ull * (N - k) + 14ull * (k - 1);
         pre = fuse;
-        // as in the row compression: the reduction's barrier publishes the update pass
+        // the barrier publishes the passes and W
         if (fuse) {
             block_argmax2_t(x1, y1, red, tog, wave);
             pre_cl = x1;
@@ -1102,12 +1197,6 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
         } else {
             bsync(wave);
         }
-        if (tid == 0) {
-            double wk = (-1.0 * fd_r<SQ>(Fk, puk, plk, ck)) / A1(A, k);
-            wk = ordered_prod(wk, Tk, k - 1);
-            A1(W, k) = wk;
-        }
-        if (!fuse) bsync(wave);
         if (k % 10 == 0 && M - k > 0) {
             for (;;) {
                 // the scanned rows' root data, gathered once into T1 / T2 when they fit
@@ -1125,29 +1214,32 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                     bsync(wave);
                 }
                 VI x = {0.0, 0};
-                for (int jc = 1 + tid; jc <= k; jc += NTH) {
-                    int pljc = A1(PL, jc);
-                    const RootG rc = rroot(jc);
-                    double mv = 0.0;
-                    int mi = 0;
-                    for (int i = 1; i <= L; i++) {
-                        double tt;
-                        if (sm) {
-                            tt = dd_r<SQ>(A1(PL, i + k), rroot(i + k), pljc, rc);
-                        } else if (stg) {
-                            const RootG ri = {T12[i - 1], T12[L + i - 1], T12[2 * L + i - 1], T12[3 * L + i - 1],
-                                              SQ ? T12[4 * L + i - 1] : 0.0};
-                            tt = dd_r<SQ>(A1(PL, i + k), ri, pljc, rc);
-                        } else {
-                            tt = ddq<SQ>(H, A1(PL, i + k), pljc);
+                const int G = scan_lanes(k, NTH), g = tid & (G - 1);  // as in the row compression
+                for (int jc = 1 + tid / G; jc - tid / G <= k; jc += NTH / G) {
+                    VI e = {0.0, 0};
+                    if (jc <= k) {
+                        const int pljc = A1(PL, jc);
+                        const RootG rc = rroot(jc);
+                        for (int i = 1 + g; i <= L; i += G) {
+                            double tt;
+                            if (sm) {
+                                tt = dd_r<SQ>(A1(PL, i + k), rroot(i + k), pljc, rc);
+                            } else if (stg) {
+                                const RootG ri = {T12[i - 1], T12[L + i - 1], T12[2 * L + i - 1], T12[3 * L + i - 1],
+                                                  SQ ? T12[4 * L + i - 1] : 0.0};
+                                tt = dd_r<SQ>(A1(PL, i + k), ri, pljc, rc);
+                            } else {
+                                tt = ddq<SQ>(H, A1(PL, i + k), pljc);
+                            }
+                            e = vi_better(e, VI{fabs(A1(Z, k + i) / tt), i});
                         }
-                        double v = fabs(A1(Z, k + i) / tt);
-                        if (mi == 0 || v > mv) { mv = v; mi = i; }
                     }
-                    VI c = {mv * fabs(A1(W, jc)), jc};
-                    VI nb = vi_better(x, c);
-                    if (nb.i == jc) IP[jc - 1] = (short)mi;
-                    x = nb;
+                    e = group_argmax(e, G);
+                    if (jc <= k) {
+                        const VI nb = vi_better(x, VI{e.v * fabs(A1(W, jc)), jc});
+                        if (nb.i == jc && g == 0) IP[jc - 1] = (short)e.i;
+                        x = nb;
+                    }
                 }
                 VI win = block_argmax_t(x, red, tog, wave);
                 if (!(win.v > rho)) break;
@@ -1197,20 +1289,16 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                     }
                     A1(Z, jj) = uj;
                     A1(W, ii) = wi;
-                    int u = A1(PL, ii); A1(PL, ii) = A1(PL, jj); A1(PL, jj) = u;
-                    short q = A1(PQ, ii); A1(PQ, ii) = A1(PQ, jj); A1(PQ, jj) = q;
-                    swapr(ii, jj);
-                    double t = A1(Dr, ii); A1(Dr, ii) = A1(Dr, jj); A1(Dr, jj) = t;
-                    t = A1(A, ii); A1(A, ii) = A1(A, jj); A1(A, jj) = t;
+                    swapr(ii, jj, false);
                 }
                 bsync(wave);
             }
         }
     }
     // ---- V generator (CauchylikeEigQ2, columns back to the node order)
+    for (int i = 1 + tid; i <= M; i += NTH) IP[A1(PQ, i) - 1] = (short)i;  // invp
     if (tid == 0) {
         atomicAdd(H.flops, fl);
-        for (int i = 1; i <= M; i++) IP[A1(PQ, i) - 1] = i;
         if (Rk < mn) {
             s_Rk = Rk;
             s_off = arena_take(H, (long)(Rk > 0 ? Rk : 1) * M);
