@@ -76,7 +76,9 @@ struct M2hCopy {
     long dst;
 };
 __global__ void k_m2h_gather(const M2hJob *, const double *, long, double *);
-__global__ void k_m2h_svd(const M2hJob *, double *, double *, double, int *, int *);
+#define M2H_SVD_WG 1024     // threads per block of k_m2h_svd
+#define M2H_LDS 19800       // LDS doubles it may take (160 KB less its static arrays)
+__global__ void k_m2h_svd(const M2hJob *, double *, double *, double, int *, int *, int);
 __global__ void k_m2h_sketch(const M2hJob *, const M2hJob *, const double *, double *, unsigned long long);
 __global__ void k_m2h_rows(const M2hBlk *, int, const M2hJob *, const double *, const double *, long, int, double *,
                            long);
@@ -2852,8 +2854,11 @@ static int mat2hss_build(hsdc_ctx *c, const double *dA, int n, int ni, double to
         if (any_sketch)
             hipLaunchKernelGGL(k_m2h_sketch, dim3(32, (unsigned)jobs.size()), dim3(WGS), 0, s, (const M2hJob *)dj,
                                (const M2hJob *)dk, (const double *)S, S, seed);
-        hipLaunchKernelGGL(k_m2h_svd, dim3((unsigned)jobs.size()), dim3(WGS), 0, s, (const M2hJob *)dk, S, Bs, tol,
-                           drank, derr);
+        long need = 0;  // LDS of the largest side's R and V
+        for (const M2hJob &J : sk) need = std::max(need, (long)J.m * std::min(J.m, J.w) + (J.w >= J.m ? (long)J.m * J.m : 0));
+        const int ldsn = (int)std::min(need, (long)M2H_LDS);
+        hipLaunchKernelGGL(k_m2h_svd, dim3((unsigned)jobs.size()), dim3(M2H_SVD_WG), sizeof(double) * (size_t)ldsn, s,
+                           (const M2hJob *)dk, S, Bs, tol, drank, derr, ldsn);
         HK(hipGetLastError());
         std::vector<int> rk(jobs.size());
         int err = 0;

@@ -29,12 +29,6 @@
 
 namespace {
 
-__device__ __forceinline__ double m2h_wsum(double v)
-{
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
 __device__ __forceinline__ int m2h_rr(int slot, int r, int P)
 {
     if (slot == 0) return 0;
@@ -85,128 +79,90 @@ __global__ __launch_bounds__(MWG) void k_m2h_gather(const M2hJob *jobs, const do
 // orthogonalised; the basis = the normalised columns by descending norm (the rest zero).
 // A pair rotates when |c_a . c_b| > L eps |c_a| |c_b|, L the column length; 60 sweeps at
 // most (else *err is set).  rank[job] = the count of singular values above tol.
+//
+// The bound is the latency of the sweeps: m - 1 rounds of m / 2 pairs, about ten sweeps,
+// each pair three dot products and a chain of square roots and divides.  Sixteen
+// wavefronts take a pair each, and R and V stay in LDS as far as lds_cap doubles hold
+// them (R and V up to m = 99, R alone up to m = 140, else global memory).  With four
+// wavefronts and R and V in global memory a level of the n = 2000, leaf 64 matrix took
+// 26 ms.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(MWG) void k_m2h_svd(const M2hJob *jobs, double *S, double *Bs, double tol, int *rank,
-                                                 int *err)
+#define M2H_SVD_WG 1024
+
+typedef __attribute__((address_space(3))) double m2h_ldbl;
+typedef __attribute__((address_space(1))) double m2h_gdbl;
+
+// Jacobi on the P columns of R (length m, ld m), with V when qr; then the singular values
+// (column norms) to sv, their descending order (ties by index) to ord, the basis to B.
+// Returns false when the sweeps did not converge.
+template <class RP, class VP>
+__device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, double *sv, int *ord, double *B,
+                                           int *s_rot)
 {
-    __shared__ double red[MWG / 64];
-    __shared__ int s_rot, perm_dummy;
-    const M2hJob J = jobs[blockIdx.x];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, NW = MWG / 64;
-    const int w = J.w, m = J.m;
-    double *T = S + J.toff, *R = T + (long)w * m, *V = R + (long)m * m;
-    double *B = Bs + J.boff, *sv = B + (long)m * m;
-    const bool qr = w >= m;
-    const int L = m, P = qr ? m : w;  // columns of length L to orthogonalise
-    (void)perm_dummy;
-    if (qr) {
-        for (int k = 0; k < m; k++) {
-            double *x = T + k + (long)k * w;
-            const int len = w - k;
-            double part = 0.0;
-            for (int i = 1 + tid; i < len; i += MWG) part += x[i] * x[i];
-            part = m2h_wsum(part);
-            if (lane == 0) red[wv] = part;
-            __syncthreads();
-            double xn = 0.0;
-            for (int q = 0; q < NW; q++) xn += red[q];
-            xn = sqrt(xn);
-            const double alpha = x[0];
-            __syncthreads();
-            if (xn == 0.0) continue;  // uniform: H = I
-            const double beta = -copysign(hypot(alpha, xn), alpha);
-            const double tau = (beta - alpha) / beta, scal = 1.0 / (alpha - beta);
-            for (int i = 1 + tid; i < len; i += MWG) x[i] *= scal;
-            __syncthreads();
-            for (int j = k + 1 + wv; j < m; j += NW) {
-                double *c = T + k + (long)j * w;
-                double d = 0.0;
-                for (int i = 1 + lane; i < len; i += 64) d += x[i] * c[i];
-                d = m2h_wsum(d);
-                d = (c[0] + d) * tau;
-                if (lane == 0) c[0] -= d;
-                for (int i = 1 + lane; i < len; i += 64) c[i] -= d * x[i];
-            }
-            __syncthreads();
-            if (tid == 0) x[0] = beta;
-            __syncthreads();
-        }
-        for (long e = tid; e < (long)m * m; e += MWG) {
-            const int i = (int)(e % m), j = (int)(e / m);
-            R[e] = (i <= j) ? T[i + (long)j * w] : 0.0;
-            V[e] = (i == j) ? 1.0 : 0.0;
-        }
-    } else {
-        for (long e = tid; e < (long)m * w; e += MWG) {
-            const int i = (int)(e % m), j = (int)(e / m);  // R area as m x w: column j = row j of T
-            R[i + (long)j * m] = T[j + (long)i * w];
-        }
-    }
-    __syncthreads();
-    const int PP = P + (P & 1);
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, NW = M2H_SVD_WG / 64;
+    const int L = m, PP = P + (P & 1);
     bool conv = P < 2;
     for (int sweep = 0; sweep < 60 && !conv; sweep++) {
-        if (tid == 0) s_rot = 0;
+        if (tid == 0) *s_rot = 0;
         __syncthreads();
+        bool rot = false;
         for (int r = 0; r < PP - 1; r++) {
             for (int pr = wv; pr < PP / 2; pr += NW) {
                 int a = m2h_rr(pr, r, PP), b = m2h_rr(PP - 1 - pr, r, PP);
                 if (a > b) { const int t = a; a = b; b = t; }
                 if (b >= P) continue;  // uniform over the wavefront
-                double *ca = R + (long)a * m, *cb = R + (long)b * m;
+                const RP ca = R + (long)a * m, cb = R + (long)b * m;
                 double al = 0.0, be = 0.0, ga = 0.0;
                 for (int k = lane; k < L; k += 64) {
                     const double x = ca[k], y = cb[k];
                     al += x * x; be += y * y; ga += x * y;
                 }
-                al = m2h_wsum(al); be = m2h_wsum(be); ga = m2h_wsum(ga);
+                al = team_bfly(al, 64); be = team_bfly(be, 64); ga = team_bfly(ga, 64);
                 if (ga == 0.0 || !(fabs(ga) > L * HSDC_EPS * sqrt(al * be))) continue;
                 const double ze = (be - al) / (2.0 * ga);
                 const double t = (ze >= 0.0 ? 1.0 : -1.0) / (fabs(ze) + sqrt(1.0 + ze * ze));
                 const double cc = 1.0 / sqrt(1.0 + t * t), ss = cc * t;
+                // columns parallel to the last bit (a block of exact rank one): every sweep
+                // shrinks the smaller one by about eps until its square underflows and the
+                // angle vanishes; a rotation that changes nothing is not counted
+                if (ss == 0.0) continue;
                 for (int k = lane; k < L; k += 64) {
                     const double x = ca[k], y = cb[k];
                     ca[k] = cc * x - ss * y;
                     cb[k] = ss * x + cc * y;
                 }
                 if (qr) {
-                    double *va = V + (long)a * m, *vb = V + (long)b * m;
+                    const VP va = V + (long)a * m, vb = V + (long)b * m;
                     for (int k = lane; k < m; k += 64) {
                         const double x = va[k], y = vb[k];
                         va[k] = cc * x - ss * y;
                         vb[k] = ss * x + cc * y;
                     }
                 }
-                if (lane == 0) atomicAdd(&s_rot, 1);
+                rot = true;
             }
             __syncthreads();
         }
-        conv = (s_rot == 0);
+        if (rot && lane == 0) *s_rot = 1;
+        __syncthreads();
+        conv = (*s_rot == 0);
         __syncthreads();
     }
-    if (!conv && tid == 0) atomicOr(err, 1);
-    // singular values (column norms), descending with ties by index; basis columns
     for (int j = wv; j < P; j += NW) {
         double q = 0.0;
         for (int k = lane; k < L; k += 64) q += R[k + (long)j * m] * R[k + (long)j * m];
-        q = sqrt(m2h_wsum(q));
+        q = sqrt(team_bfly(q, 64));
         if (lane == 0) sv[j] = q;
     }
     __syncthreads();
-    int *ord = (int *)(sv + m);  // P ints after the singular values
-    if (tid == 0) {
-        for (int j = 0; j < P; j++) ord[j] = j;
-        for (int i = 0; i + 1 < P; i++) {
-            int k = i;
-            for (int j = i + 1; j < P; j++) if (sv[ord[j]] > sv[ord[k]]) k = j;
-            const int t = ord[i]; ord[i] = ord[k]; ord[k] = t;
-        }
-        int cnt = 0;
-        for (int j = 0; j < P; j++) cnt += sv[ord[j]] > tol;
-        rank[blockIdx.x] = cnt;
+    for (int j = tid; j < P; j += M2H_SVD_WG) {
+        const double x = sv[j];
+        int rk = 0;
+        for (int i = 0; i < P; i++) rk += (sv[i] > x || (sv[i] == x && i < j)) ? 1 : 0;
+        ord[rk] = j;
     }
     __syncthreads();
-    for (long e = tid; e < (long)m * m; e += MWG) {
+    for (long e = tid; e < (long)m * m; e += M2H_SVD_WG) {
         const int i = (int)(e % m), j = (int)(e / m);
         double v = 0.0;
         if (j < P) {
@@ -219,6 +175,83 @@ __global__ __launch_bounds__(MWG) void k_m2h_svd(const M2hJob *jobs, double *S, 
         }
         B[e] = v;
     }
+    return conv;
+}
+
+__global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_svd(const M2hJob *jobs, double *S, double *Bs, double tol, int *rank,
+                                                        int *err, int lds_cap)
+{
+    extern __shared__ double m2h_dyn[];  // lds_cap doubles
+    __shared__ double red[M2H_SVD_WG / 64];
+    __shared__ int s_rot, s_cnt;
+    const M2hJob J = jobs[blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, NW = M2H_SVD_WG / 64;
+    const int w = J.w, m = J.m;
+    double *T = S + J.toff, *Rg = T + (long)w * m, *Vg = Rg + (long)m * m;
+    double *B = Bs + J.boff, *sv = B + (long)m * m;
+    int *ord = (int *)(sv + m);  // P ints after the singular values
+    const bool qr = w >= m;
+    const int P = qr ? m : w;  // columns of length m to orthogonalise
+    const long rsz = (long)m * P;
+    const bool rl = rsz <= lds_cap, vl = rl && qr && rsz + (long)m * m <= lds_cap;
+    m2h_ldbl *Rl = (m2h_ldbl *)m2h_dyn, *Vl = Rl + rsz;
+    if (qr) {
+        for (int k = 0; k < m; k++) {
+            double *x = T + k + (long)k * w;
+            const int len = w - k;
+            double part = 0.0;
+            for (int i = 1 + tid; i < len; i += M2H_SVD_WG) part += x[i] * x[i];
+            part = team_bfly(part, 64);
+            if (lane == 0) red[wv] = part;
+            __syncthreads();
+            double xn = 0.0;
+            for (int q = 0; q < NW; q++) xn += red[q];
+            xn = sqrt(xn);
+            const double alpha = x[0];
+            __syncthreads();
+            if (xn == 0.0) continue;  // uniform: H = I
+            const double beta = -copysign(hypot(alpha, xn), alpha);
+            const double tau = (beta - alpha) / beta, scal = 1.0 / (alpha - beta);
+            for (int i = 1 + tid; i < len; i += M2H_SVD_WG) x[i] *= scal;
+            __syncthreads();
+            for (int j = k + 1 + wv; j < m; j += NW) {
+                double *c = T + k + (long)j * w;
+                double d = 0.0;
+                for (int i = 1 + lane; i < len; i += 64) d += x[i] * c[i];
+                d = team_bfly(d, 64);
+                d = (c[0] + d) * tau;
+                if (lane == 0) c[0] -= d;
+                for (int i = 1 + lane; i < len; i += 64) c[i] -= d * x[i];
+            }
+            __syncthreads();
+            if (tid == 0) x[0] = beta;
+            __syncthreads();
+        }
+        for (long e = tid; e < (long)m * m; e += M2H_SVD_WG) {
+            const int i = (int)(e % m), j = (int)(e / m);
+            const double r = (i <= j) ? T[i + (long)j * w] : 0.0, v = (i == j) ? 1.0 : 0.0;
+            if (rl) Rl[e] = r; else Rg[e] = r;
+            if (vl) Vl[e] = v; else Vg[e] = v;
+        }
+    } else {
+        for (long e = tid; e < rsz; e += M2H_SVD_WG) {
+            const int i = (int)(e % m), j = (int)(e / m);  // R area as m x w: column j = row j of T
+            const double r = T[j + (long)i * w];
+            if (rl) Rl[e] = r; else Rg[e] = r;
+        }
+    }
+    if (tid == 0) s_cnt = 0;
+    __syncthreads();
+    bool conv;
+    m2h_gdbl *Rq = (m2h_gdbl *)Rg, *Vq = (m2h_gdbl *)Vg;
+    if (vl) conv = m2h_jacobi(Rl, Vl, qr, m, P, sv, ord, B, &s_rot);
+    else if (rl) conv = m2h_jacobi(Rl, Vq, qr, m, P, sv, ord, B, &s_rot);
+    else conv = m2h_jacobi(Rq, Vq, qr, m, P, sv, ord, B, &s_rot);
+    if (!conv && tid == 0) atomicOr(err, 1);
+    for (int j = tid; j < P; j += M2H_SVD_WG)
+        if (sv[j] > tol) atomicAdd(&s_cnt, 1);
+    __syncthreads();
+    if (tid == 0) rank[blockIdx.x] = s_cnt;
 }
 
 // ---------------------------------------------------------------------------
