@@ -1544,14 +1544,14 @@ __global__ __launch_bounds__(WG) void k_bgemm(const BG *items)
             const double *bp = Bs + (kq + lk) * BG_BP + lr;
             const double a0 = ap[0], a1 = ap[16];
             const double b0 = bp[0], b1 = bp[16], b2 = bp[32], b3 = bp[48];
-            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-            acc[0][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b2, acc[0][2], 0, 0, 0);
-            acc[0][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b3, acc[0][3], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-            acc[1][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b2, acc[1][2], 0, 0, 0);
-            acc[1][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b3, acc[1][3], 0, 0, 0);
+            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(b0, a0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(b1, a0, acc[0][1], 0, 0, 0);
+            acc[0][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(b2, a0, acc[0][2], 0, 0, 0);
+            acc[0][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(b3, a0, acc[0][3], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(b0, a1, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(b1, a1, acc[1][1], 0, 0, 0);
+            acc[1][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(b2, a1, acc[1][2], 0, 0, 0);
+            acc[1][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(b3, a1, acc[1][3], 0, 0, 0);
         }
         __syncthreads();  // every wavefront is done with this chunk
         if (more) {
@@ -1559,17 +1559,19 @@ __global__ __launch_bounds__(WG) void k_bgemm(const BG *items)
             __syncthreads();
         }
     }
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 4; b++) {
-            const int col = c0 + b * 16 + lr;
+    // The B fragment is the MFMA's first operand, so that a lane's four results lie along a
+    // row of C (columns lk, lk + 4, ...) and the 16 lanes of a store hold 16 adjacent
+    // rows: each store writes 128-byte runs of C's columns, not 32-byte ones.  The
+    // products and their order are the same.
+    for (int b = 0; b < 4; b++)
+        for (int i = 0; i < 4; i++) {
+            const int col = c0 + b * 16 + lk + 4 * i;
             if (col >= g.n) continue;
             const long pc = g.cmap ? (long)((const __attribute__((address_space(1))) int *)g.cmap)[col] - g.cmoff : (long)col;
-            for (int i = 0; i < 4; i++) {
-                int row = rb + wr + a * 16 + lk + 4 * i;
-                if (row < g.nrow) {
-                    gdblw *cp = (gdblw *)g.C + ((long)row + pc * g.ldc);
-                    *cp = g.beta ? (*cp + acc[a][b][i]) : acc[a][b][i];
-                }
+            gdblw *cp = (gdblw *)g.C + pc * g.ldc;
+            for (int a = 0; a < 2; a++) {
+                const int row = rb + wr + a * 16 + lr;
+                if (row < g.nrow) cp[row] = g.beta ? (cp[row] + acc[a][b][i]) : acc[a][b][i];
             }
         }
 }
@@ -1680,7 +1682,7 @@ __global__ __launch_bounds__((BM / (16 * TA)) * (BN / (16 * TB)) * 64) void k_bg
             for (int a = 0; a < TA; a++)
 #pragma unroll
                 for (int b = 0; b < TB; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
+                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b], av[a], acc[a][b], 0, 0, 0);
         }
         if (DB) {
             // the other slab was last read before the previous barrier: fill it now, then
@@ -1700,20 +1702,19 @@ __global__ __launch_bounds__((BM / (16 * TA)) * (BN / (16 * TB)) * 64) void k_bg
             }
         }
     }
+    // first operand B, as in k_bgemm: 128-byte runs of C's columns per store
 #pragma unroll
-    for (int a = 0; a < TA; a++)
+    for (int b = 0; b < TB; b++)
 #pragma unroll
-        for (int b = 0; b < TB; b++) {
-            const int col = c0 + wc + b * 16 + lr;
+        for (int i = 0; i < 4; i++) {
+            const int col = c0 + wc + b * 16 + lk + 4 * i;
             if (col >= g.n) continue;
             const long pc = g.cmap ? (long)((const __attribute__((address_space(1))) int *)g.cmap)[col] - g.cmoff : (long)col;
+            gdblw *cp = (gdblw *)g.C + pc * g.ldc;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = rb + wr + a * 16 + lk + 4 * i;
-                if (row < g.nrow) {
-                    gdblw *cp = (gdblw *)g.C + ((long)row + pc * g.ldc);
-                    *cp = g.beta ? (*cp + acc[a][b][i]) : acc[a][b][i];
-                }
+            for (int a = 0; a < TA; a++) {
+                const int row = rb + wr + a * 16 + lr;
+                if (row < g.nrow) cp[row] = g.beta ? (cp[row] + acc[a][b][i]) : acc[a][b][i];
             }
         }
 }
