@@ -19,6 +19,7 @@
 
 #define WG 256
 #define A1(a, i) (a)[(i) - 1]
+#define HSS_RB 2  // outside columns a thread takes at a time in the RRLU passes
 
 // Pointers typed by address space: global memory (1) and LDS (3).  Loads through an
 // untyped pointer compile to FLAT instructions, which the compiler must order against
@@ -161,7 +162,7 @@ __device__ __forceinline__ double lane_value(double v, int l)
     const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-// The (value, smallest index) maximum over the wavefront's first NL lanes (64 or 8), in
+// The (value, smallest index) maximum over the wavefront's first NL lanes (4 to 64), in
 // every lane, for values >= 0: the values go through a prefix of DPP moves (no LDS
 // traffic), the index is read from the lane a ballot finds.  A butterfly of (value,
 // index) pairs, three of whose six steps cross lanes through LDS, took about 1000 cycles
@@ -172,9 +173,9 @@ __device__ __forceinline__ VI wave_argmax(VI x)
     const double v = x.i > 0 ? x.v : -1.0;
     double m = dpp_max<0x111>(v);  // row_shr:1
     m = dpp_max<0x112>(m);
-    m = dpp_max<0x114>(m);
-    if (NL == 64) {
-        m = dpp_max<0x118>(m);
+    if (NL > 4) m = dpp_max<0x114>(m);
+    if (NL > 8) m = dpp_max<0x118>(m);
+    if (NL > 16) {
         m = dpp_max<0x142>(m);  // row_bcast:15
         m = dpp_max<0x143>(m);  // row_bcast:31
     }
@@ -191,37 +192,36 @@ __device__ __forceinline__ VI wave_argmax(VI x)
     }
     return VI{lane_value(x.v, l), i};
 }
-// Over the block with one barrier: successive calls alternate between the two halves of
-// sh (4 x blockDim / 64 entries; a half holds 2 x blockDim / 64 so that the two-value
-// form below shares them), so a call's writes never meet the previous call's reads
-// and the trailing barrier that protects a single buffer is not needed.  tog is
-// uniform over the block and flips on every call.  Blocks of 4 or 8 wavefronts.
-// With wave set the block is one wavefront, and nothing goes through sh.
-__device__ __forceinline__ VI block_argmax_t(VI x, VI *sh, int &tog, bool wave = false)
+// Over the block of NW (up to 16) wavefronts with one barrier: successive calls alternate
+// between the two halves of sh (4 NW entries; a half holds 2 NW so that the two-value form
+// below shares them), so a call's writes never meet the previous call's reads and the
+// trailing barrier that protects a single buffer is not needed.  tog is uniform over the
+// block and flips on every call.
+template <int NW>
+__device__ __forceinline__ VI block_argmax_t(VI x, VI *sh, int &tog)
 {
-    const int tid = threadIdx.x, nw = (int)(blockDim.x >> 6);
-    VI *b = sh + tog * 2 * nw;
+    const int tid = threadIdx.x;
+    VI *b = sh + tog * 2 * NW;
     tog ^= 1;
     x = wave_argmax<64>(x);
-    if (wave) return x;
     if ((tid & 63) == 0) b[tid >> 6] = x;
     __syncthreads();
-    return wave_argmax<8>(b[tid & (nw - 1)]);
+    return wave_argmax<NW>(b[tid & (NW - 1)]);
 }
 // Two independent (value, index) maxima under one barrier, in the same alternating
 // halves of sh.
-__device__ __forceinline__ void block_argmax2_t(VI &x, VI &y, VI *sh, int &tog, bool wave = false)
+template <int NW>
+__device__ __forceinline__ void block_argmax2_t(VI &x, VI &y, VI *sh, int &tog)
 {
-    const int tid = threadIdx.x, nw = (int)(blockDim.x >> 6);
-    VI *b = sh + tog * 2 * nw;
+    const int tid = threadIdx.x;
+    VI *b = sh + tog * 2 * NW;
     tog ^= 1;
     x = wave_argmax<64>(x);
     y = wave_argmax<64>(y);
-    if (wave) return;
-    if ((tid & 63) == 0) { b[tid >> 6] = x; b[nw + (tid >> 6)] = y; }
+    if ((tid & 63) == 0) { b[tid >> 6] = x; b[NW + (tid >> 6)] = y; }
     __syncthreads();
-    x = wave_argmax<8>(b[tid & (nw - 1)]);
-    y = wave_argmax<8>(b[nw + (tid & (nw - 1))]);
+    x = wave_argmax<NW>(b[tid & (NW - 1)]);
+    y = wave_argmax<NW>(b[NW + (tid & (NW - 1))]);
 }
 // lanes per column of the swap check's scan: the k columns' rows are spread over all NTH
 // threads, G (a power of two) to a column
@@ -242,17 +242,12 @@ __device__ __forceinline__ VI group_argmax(VI x, int g)
     if (g > 1) x = vi_step<1>(x);
     return x;
 }
-// The block's barrier, or for a one-wavefront block the ordering of its LDS accesses
-// (a wavefront executes in lockstep; the fence completes lane 0's writes before any
-// lane reads them).
-__device__ __forceinline__ void bsync(bool wave)
+// Orders a wavefront's own LDS accesses (it executes in lockstep; the fence completes
+// its lanes' writes before any lane reads them)
+__device__ __forceinline__ void wsync()
 {
-    if (wave) {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-    } else {
-        __syncthreads();
-    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
 }
 // x * t[0] * t[1] * ... * t[n - 1], multiplied in that order (one thread), with the
 // factors read from LDS eight at a time ahead of their multiplications
@@ -312,13 +307,18 @@ __device__ __forceinline__ long scratch_take(const HssMerge &H, long n)
 // rows: the node's M row generators (LDS); columns: the N column generators
 // outside the node (private copies: V in LDS when it fits, else global; PU global,
 // with positions 1..min(M, N) mirrored in LDS).
-// The passes over the N columns take RB columns per thread at a time (7, or 6 in the
-// squared form, for 512 threads; 4 for 256, whose launches put several workgroups on a
-// CU): the loads of all RB (V, PU, then the roots' gathered values) are issued before
-// any result is used, the next batch's V and PU before the current batch's results,
-// and the stores of a batch after its loads.  A step the swap check does not follow runs the next step's
-// row search inside its own row update and reduces it with the next step's first
-// column search under one barrier.
+// The passes over the N columns take HSS_RB = 2 columns per thread at a time: the loads of
+// both (V, PU, then the roots' gathered values) are issued before any result is used, the
+// next two's V and PU before the current results, and the stores after the loads.  The
+// width is bounded by the code, not the registers: a step runs through four such passes
+// and two searches, every one an inlined body, and with 7 columns (8 in the column
+// compression) the kernels were 59-66 KB, as much as the instruction cache two CUs share
+// (64 KB); with 2 they are 38-45 KB.  A pivot step of a node with 240 outside columns
+// went from 17 to 11 thousand cycles, of one with 4000 from 33 to 27 thousand.  Widths 3
+// and 4 are 1-3 % slower overall, 1024 threads 5-17 %, 256 threads 4-8 %; one wavefront
+// for small nodes, without barriers, lost to the block once its reductions were short.
+// A step the swap check does not follow runs the next step's row search inside its own
+// row update and reduces it with the next step's first column search under one barrier.
 // ---------------------------------------------------------------------------
 template <int HSS_CWG, bool SQ>
 __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, const HssNode *nodes, int nn,
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
     __shared__ long s_off;
     __shared__ int s_M, s_N, s_Rk, s_flag, s_ii, s_jj;
     const int tid = threadIdx.x, lane = tid & 63;
-    constexpr int RB = HSS_CWG >= 512 ? (SQ ? 6 : 7) : 4;  // within 256 VGPRs
+    constexpr int RB = HSS_RB;
     if ((int)blockIdx.x >= nn) return;
     HssNode Nd = nodes[blockIdx.x];
     const HssMerge H = hm[Nd.mrg];
@@ -369,11 +369,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
     const bool vl = N <= lds_cap;   // all three uniform over the block
     const bool pl = (long)N + (N + 1) / 2 <= lds_cap;
     const bool sm = (long)N * (1 + RD) + (N + 1) / 2 <= lds_cap;
-    // A node whose data all sit in LDS and whose outside part is small runs on one
-    // wavefront: its steps need no block barrier (the other waves leave here)
-    const bool wave = sm && N <= 384;
-    if (wave && tid >= 64) return;
-    const int NTH = wave ? 64 : HSS_CWG;
+    constexpr int NTH = HSS_CWG;
     ldbl *Vl = (ldbl *)hss_dyn;
     ldbl *Rl = Vl + NS;  // sm: f0, f1, dl, dr (and s) of every column, NS apart
     __attribute__((address_space(3))) int *PUl =
@@ -445,9 +441,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
             v[u] = vld(j);
         }
     };
-    // one batch with the roots' values (CP scan)
-    auto bload = [&](int j0, int *pw, double *v, RootG *c) {
-        cload(j0, pw, v);
+    // the columns' root values, from LDS or gathered
+    auto rload = [&](int j0, const int *pw, RootG *c) {
         #pragma unroll
         for (int u = 0; u < RB; u++) c[u] = sm ? rl_get(min(j0 + u * NTH, N)) : root_load<SQ>(H, pw[u]);
     };
@@ -522,7 +517,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         PQ[i] = (short)(i + 1);
         W[i] = 0.0;
     }
-    bsync(wave);
+    __syncthreads();
     double amax = 0.0;
     int Rk = mn;
     const double rho = 1.5;
@@ -548,7 +543,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                 cw = croot(k);
                 cl = rowsearch(k, pwk, cw);
                 rw = colsearch(k, A1(PL, k), A1(F, k));
-                block_argmax2_t(cl, rw, red, tog, wave);
+                block_argmax2_t<HSS_CWG / 64>(cl, rw, red, tog);
             }
             double junkL = cl.v * fabs(vld(k)), junkU = rw.v * fabs(A1(Z, k));
             double piv = fabs(A1(Z, k) * vld(k) / fd_r<SQ>(A1(F, k), A1(PL, k), A1(PUs, k), cw));
@@ -558,27 +553,27 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                 // Every thread has read position k for the tests above before any swap: a
                 // row swap is made after the column search it feeds (which reads the
                 // incoming row where it still is) and its reduction's barrier.
-                if (flg == 0) bsync(wave);
+                if (flg == 0) __syncthreads();
                 for (;;) {
                     if (flg == 1) {
                         const int jr = jjL + k - 1;
-                        jjU = block_argmax_t(colsearch(k, A1(PL, jr), A1(F, jr)), red, tog, wave).i;
+                        jjU = block_argmax_t<HSS_CWG / 64>(colsearch(k, A1(PL, jr), A1(F, jr)), red, tog).i;
                         fl += 4ull * (N - k + 1);
                         if (tid == 0) swapr(k, jr);
                         if (jjU == 1) {
-                            bsync(wave);
+                            __syncthreads();
                             break;
                         }
                     }
                     if (tid == 0) swapc(k, jjU + k - 1);
-                    bsync(wave);
+                    __syncthreads();
                     const int pwk2 = A1(PUs, k);
                     cw = croot(k);
                     const bool few = M - k < 256;
-                    jjL = few ? rowsearch_w(k, pwk2, cw).i : block_argmax_t(rowsearch(k, pwk2, cw), red, tog, wave).i;
+                    jjL = few ? rowsearch_w(k, pwk2, cw).i : block_argmax_t<HSS_CWG / 64>(rowsearch(k, pwk2, cw), red, tog).i;
                     fl += 4ull * (M - k + 1);
                     if (jjL == 1) {
-                        if (few) bsync(wave);  // before the update pass writes what the search reads
+                        if (few) __syncthreads();  // before the update pass writes what the search reads
                         break;
                     }
                     flg = 1;
@@ -599,7 +594,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                 double v[RB], mv[RB];
                 int mi[RB];
                 RootG c[RB];
-                bload(j0, pw, v, c);
+                cload(j0, pw, v);
+                rload(j0, pw, c);
                 #pragma unroll
                 for (int u = 0; u < RB; u++) { mv[u] = -DBL_MAX; mi[u] = 0; }
                 for (int i = k; i <= M; i++) {
@@ -624,16 +620,16 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                     best = nb;
                 }
             }
-            VI win = block_argmax_t(best, red, tog, wave);
-            bsync(wave);
+            VI win = block_argmax_t<HSS_CWG / 64>(best, red, tog);
+            __syncthreads();
             if (win.i > 0 && best.i == win.i) { s_ii = bestrow.i; s_jj = win.i; }
-            bsync(wave);
+            __syncthreads();
             if (tid == 0) {
                 int ii = s_ii, jj = s_jj;
                 swapr(k, ii + k - 1);
                 swapc(k, jj + k - 1);
             }
-            bsync(wave);
+            __syncthreads();
             cw = croot(k);
             ukk = A1(Z, k) * vld(k) / fd_r<SQ>(A1(F, k), A1(PL, k), A1(PUs, k), cw);
             amax = fmax(amax, fabs(ukk));
@@ -661,7 +657,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                 const double t2 = -1.0 * fd_r<SQ>(Fk, plk, puj, croot(j));
                 A1(T1, j) = t2 / ppq<SQ>(A1(F, j), Fk);
             }
-            bsync(true);
+            wsync();
             if (lane == 0) A1(W, k) = ordered_prod(fd_r<SQ>(Fk, plk, puk, ck) / A1(A, k), T1, k - 1);
         }
         VI x1 = {0.0, 0};
@@ -687,12 +683,12 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         pre = fuse;
         // The reduction's barrier (or the one before a swap check) publishes the passes and W
         if (fuse) {
-            block_argmax2_t(x1, y1, red, tog, wave);
+            block_argmax2_t<HSS_CWG / 64>(x1, y1, red, tog);
             pre_cl = x1;
             pre_rw = y1;
             cnext = cn;
         } else {
-            bsync(wave);
+            __syncthreads();
         }
         // ---- every 10 steps: swap while max |Mat_N| > rho (searchMax2Eig)
         if (k % 10 == 0 && M - k > 0) {
@@ -715,11 +711,11 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                         x = nb;
                     }
                 }
-                VI win = block_argmax_t(x, red, tog, wave);
+                VI win = block_argmax_t<HSS_CWG / 64>(x, red, tog);
                 if (!(win.v > rho)) break;
                 const int ii = win.i, jj = IP[ii - 1] + k;
                 fl += 10ull * (N - k) + 8ull * M + 18ull * k;
-                bsync(wave);
+                __syncthreads();
                 const double Fii = A1(F, ii), Fjj = A1(F, jj);
                 const int plii = A1(PL, ii), pljj = A1(PL, jj);
                 cpass(k + 1, [&](int j, int pw, double v, const RootG &c) {
@@ -742,7 +738,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                     temp = -1.0 * fd_r<SQ>(Fjj, pljj, puj, cj);
                     A1(T2, j) = temp / ppq<SQ>(A1(F, j), Fjj);
                 }
-                bsync(wave);
+                __syncthreads();
                 if (tid == 0) {
                     const int puii = A1(PUs, ii);
                     const RootG cii = croot(ii);
@@ -760,7 +756,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
                     double t = A1(F, ii); A1(F, ii) = A1(F, jj); A1(F, jj) = t;
                     t = A1(A, ii); A1(A, ii) = A1(A, jj); A1(A, jj) = t;
                 }
-                bsync(wave);
+                __syncthreads();
             }
         }
     }
@@ -780,7 +776,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
         H.usz[2 * (node - 1) + 1] = s_Rk;
         H.pu[node - 1] = s_off;
     }
-    bsync(wave);
+    __syncthreads();
     const long off = s_off;
     if (off >= 0) {
         double *Ug = H.arena + off;
@@ -832,7 +828,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
     __shared__ long s_off;
     __shared__ int s_M, s_N, s_Rk, s_flag, s_ii, s_jj;
     const int tid = threadIdx.x, lane = tid & 63;
-    constexpr int RB = HSS_CWG >= 512 ? 8 : 4;
+    constexpr int RB = HSS_RB;
     if ((int)blockIdx.x >= nn) return;
     HssNode Nd = nodes[blockIdx.x];
     const HssMerge H = hm[Nd.mrg];
@@ -862,11 +858,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
     const bool vl = N <= lds_cap;  // all three uniform over the block
     const bool pl = (long)N + (N + 1) / 2 <= lds_cap;
     const bool sm = 2L * N + (N + 1) / 2 + (long)RD * M <= lds_cap;
-    // A node whose data all sit in LDS and whose outside part is small runs on one
-    // wavefront: its steps need no block barrier (the other waves leave here)
-    const bool wave = sm && N <= 384;
-    if (wave && tid >= 64) return;
-    const int NTH = wave ? 64 : HSS_CWG;
+    constexpr int NTH = HSS_CWG;
     ldbl *Vl = (ldbl *)hss_dyn;
     ldbl *FFl = Vl + NS;     // sm: FF(PU(j))
     ldbl *RRl = FFl + NS;    // sm: f0, f1, dl, dr (and s) of the node's M columns, M apart
@@ -939,8 +931,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
             v[u] = vld(j);
         }
     };
-    auto bload = [&](int j0, int *pd, double *v, double *ffd) {
-        cload(j0, pd, v);
+    auto fload = [&](int j0, const int *pd, double *ffd) {
         #pragma unroll
         for (int u = 0; u < RB; u++) ffd[u] = sm ? A1(FFl, min(j0 + u * NTH, N)) : A1(FF, pd[u]);
     };
@@ -1017,7 +1008,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
             if (SQ) RRl[4 * M + i] = r.s;
         }
     }
-    bsync(wave);
+    __syncthreads();
     double amax = 0.0;
     int Rk = mn;
     const double rho = 1.5;
@@ -1046,7 +1037,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                 cr = rroot(k);
                 cl = rowsearch(k, puk, ffp);
                 rw = colsearch(k, plk, cr);
-                block_argmax2_t(cl, rw, red, tog, wave);
+                block_argmax2_t<HSS_CWG / 64>(cl, rw, red, tog);
             }
             double junkL = cl.v * fabs(vld(k)), junkU = rw.v * fabs(A1(Z, k));
             double den;
@@ -1061,29 +1052,29 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                 int flg = (junkL > junkU) ? 1 : 0;
                 int jjL = cl.i, jjU = rw.i;
                 // barriers as in the row compression
-                if (flg == 0) bsync(wave);
+                if (flg == 0) __syncthreads();
                 for (;;) {
                     if (flg == 1) {
                         const int jr = jjL + k - 1;
                         const int plr = A1(PL, jr);
                         cr = rroot(jr);
-                        jjU = block_argmax_t(colsearch(k, plr, cr), red, tog, wave).i;
+                        jjU = block_argmax_t<HSS_CWG / 64>(colsearch(k, plr, cr), red, tog).i;
                         fl += 4ull * (N - k + 1);
                         if (tid == 0) swapr(k, jr, true);
                         if (jjU == 1) {
-                            bsync(wave);
+                            __syncthreads();
                             break;
                         }
                     }
                     if (tid == 0) swapc(k, jjU + k - 1);
-                    bsync(wave);
+                    __syncthreads();
                     const int puk2 = A1(PUs, k);
                     ffp = A1(FF, puk2);
                     const bool few = M - k < 256;
-                    jjL = few ? rowsearch_w(k, puk2, ffp).i : block_argmax_t(rowsearch(k, puk2, ffp), red, tog, wave).i;
+                    jjL = few ? rowsearch_w(k, puk2, ffp).i : block_argmax_t<HSS_CWG / 64>(rowsearch(k, puk2, ffp), red, tog).i;
                     fl += 4ull * (M - k + 1);
                     if (jjL == 1) {
-                        if (few) bsync(wave);  // before the update pass writes what the search reads
+                        if (few) __syncthreads();  // before the update pass writes what the search reads
                         break;
                     }
                     flg = 1;
@@ -1102,7 +1093,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                 int pd[RB];
                 double v[RB], ffd[RB], mv[RB];
                 int mi[RB];
-                bload(j0, pd, v, ffd);
+                cload(j0, pd, v);
+                fload(j0, pd, ffd);
                 #pragma unroll
                 for (int u = 0; u < RB; u++) { mv[u] = 0.0; mi[u] = 0; }
                 for (int i = k; i <= M; i++) {
@@ -1127,14 +1119,14 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                     best = nb;
                 }
             }
-            VI win = block_argmax_t(best, red, tog, wave);
+            VI win = block_argmax_t<HSS_CWG / 64>(best, red, tog);
             if (win.i > 0 && best.i == win.i) { s_ii = bestrow; s_jj = win.i; }
-            bsync(wave);
+            __syncthreads();
             if (tid == 0) {
                 swapr(k, s_ii + k - 1, true);
                 swapc(k, s_jj + k - 1);
             }
-            bsync(wave);
+            __syncthreads();
             cr = rroot(k);
             ffp = A1(FF, A1(PUs, k));
             ukk = A1(Z, k) * vld(k) / (-1.0 * fd_r<SQ>(ffp, A1(PUs, k), A1(PL, k), cr));
@@ -1162,7 +1154,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                 temp2 = dd_r<SQ>(plj, rj, plk, ck);
                 A1(T1, j) = temp / temp2;
             }
-            bsync(true);
+            wsync();
             if (lane == 0) A1(W, k) = ordered_prod((-1.0 * fd_r<SQ>(Fk, puk, plk, ck)) / A1(A, k), T1, k - 1);
         }
         VI x1 = {0.0, 0};
@@ -1189,13 +1181,13 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
         pre = fuse;
         // the barrier publishes the passes and W
         if (fuse) {
-            block_argmax2_t(x1, y1, red, tog, wave);
+            block_argmax2_t<HSS_CWG / 64>(x1, y1, red, tog);
             pre_cl = x1;
             pre_rw = y1;
             cnext = ck1;
             ffnext = ffn;
         } else {
-            bsync(wave);
+            __syncthreads();
         }
         if (k % 10 == 0 && M - k > 0) {
             for (;;) {
@@ -1211,7 +1203,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                         T12[3 * L + q] = r.dr;
                         if (SQ) T12[4 * L + q] = r.s;
                     }
-                    bsync(wave);
+                    __syncthreads();
                 }
                 VI x = {0.0, 0};
                 const int G = scan_lanes(k, NTH), g = tid & (G - 1);  // as in the row compression
@@ -1241,11 +1233,11 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                         x = nb;
                     }
                 }
-                VI win = block_argmax_t(x, red, tog, wave);
+                VI win = block_argmax_t<HSS_CWG / 64>(x, red, tog);
                 if (!(win.v > rho)) break;
                 const int ii = win.i, jj = IP[ii - 1] + k;
                 fl += 10ull * (N - k) + 12ull * M + 22ull * k;
-                bsync(wave);
+                __syncthreads();
                 const int plii = A1(PL, ii), pljj = A1(PL, jj);
                 const RootG cii = rroot(ii), cjj = rroot(jj);
                 cpass(k + 1, [&](int j, int pd, double v, double ffd) {
@@ -1275,7 +1267,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                     temp2 = ddq<SQ>(H, A1(PL, j), pljj);
                     A1(T2, j) = temp / temp2;
                 }
-                bsync(wave);
+                __syncthreads();
                 if (tid == 0) {
                     const int puii = A1(PUs, ii);
                     double temp = ddq<SQ>(H, plii, pljj);
@@ -1291,7 +1283,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
                     A1(W, ii) = wi;
                     swapr(ii, jj, false);
                 }
-                bsync(wave);
+                __syncthreads();
             }
         }
     }
@@ -1310,7 +1302,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
         H.vsz[2 * (node - 1) + 1] = M;
         H.pv[node - 1] = s_off;
     }
-    bsync(wave);
+    __syncthreads();
     const long off = s_off;
     if (off >= 0) {
         double *Vg = H.arena + off;
