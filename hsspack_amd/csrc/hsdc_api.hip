@@ -58,7 +58,9 @@ __global__ void k_final(const Prob *, const int *, Work, const int *, double *, 
 __global__ void k_zfill(double *, long, long, long);
 __global__ void k_dgemm_nn(int, int, int, const double *, long, const double *, long, double *, long);
 __global__ void k_transpose(int, int, const double *, long, double *, long);
-__global__ void k_cauchy2hss(C2H);
+#define C2H_WG 512     // threads of k_cauchy2hss
+#define C2H_LDS 18432  // LDS doubles it may take
+__global__ void k_cauchy2hss(C2H, int);
 struct M2hJob {
     int rs, rn, cs, cn;
     int w, m;
@@ -2604,8 +2606,8 @@ int hsdc_cauchyhssmm(hsdc_ctx *c, const double *d, const double *f, const double
     HssTree T;
     const bool tree = hss_make_tree(T, n, ni);
     const size_t nn = (size_t)n;
-    // device storage: inputs, working generators and scratch (16 n), the matrix B
-    CK(ensure(c->xb, sizeof(double) * 16 * nn));
+    // device storage: inputs, working generators and scratch (18 n), the matrix B
+    CK(ensure(c->xb, sizeof(double) * 18 * nn));
     double *gd = (double *)c->xb.p;
     const double *hsrc[4] = {d, f, u, v};
     for (int i = 0; i < 4; i++) HK(hipMemcpyAsync(gd + i * nn, hsrc[i], sizeof(double) * nn, hipMemcpyHostToDevice, s));
@@ -2665,11 +2667,13 @@ int hsdc_cauchyhssmm(hsdc_ctx *c, const double *d, const double *f, const double
         C.D = gd + 4 * nn; C.F = gd + 5 * nn; C.U = gd + 6 * nn; C.V = gd + 7 * nn;
         for (int i = 0; i < 4; i++)
             HK(hipMemcpyAsync(gd + (4 + i) * nn, gd + i * nn, sizeof(double) * nn, hipMemcpyDeviceToDevice, s));
-        C.Di = gd + 8 * nn; C.Fi = gd + 9 * nn; C.Ui = gd + 10 * nn; C.Vi = gd + 11 * nn; C.Z = gd + 12 * nn;
-        C.W = gd + 13 * nn;
-        C.PL = (int *)(gd + 14 * nn); C.PU = (int *)(gd + 15 * nn);
+        C.Fi = gd + 8 * nn; C.Vi = gd + 9 * nn; C.S = gd + 10 * nn;
+        C.PL = (int *)(gd + 16 * nn); C.PU = (int *)(gd + 17 * nn);
         HK(hipEventRecord(c->ev0, s));
-        hipLaunchKernelGGL(k_cauchy2hss, dim3(1), dim3(1024), 0, s, C);
+        // 7 doubles per row of the largest node (a leaf, or two children's skeletons) and 2
+        // per outside column; a compression that needs more takes the global scratch
+        const int ldsn = (int)std::min((long)C2H_LDS, 2L * n + 7L * 2 * *std::max_element(T.m.begin(), T.m.end()) + 2);
+        hipLaunchKernelGGL(k_cauchy2hss, dim3(1), dim3(C2H_WG), sizeof(double) * (size_t)ldsn, s, C, ldsn);
         HK(hipGetLastError());
         HK(hipEventRecord(c->ev1, s));
         // generator directory back to the host

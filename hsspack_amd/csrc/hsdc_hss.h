@@ -42,7 +42,7 @@ struct C2H {
     const int *ch;          // 2 per node: children (0, 0 for a leaf)
     const int *rng;         // 2 per node: first and last original index (1-based)
     double *D, *F, *U, *V;  // working generators (n)
-    double *Di, *Fi, *Ui, *Vi, *Z, *W;  // node scratch (n)
+    double *S, *Fi, *Vi;    // node scratch when LDS is too small: six arrays of n, then n each
     int *PL, *PU;           // permutations (n)
     int *lsr, *lsc;         // skeleton stacks (lvl + 3)
     double *arena;          // U, V, B generators

@@ -126,25 +126,6 @@ __device__ __forceinline__ VI vi_step(VI x)
     y.i = xlane32<O>(x.i);
     return vi_better(x, y);
 }
-// (value, index) maximum with ties to the smaller index is a total order, so the
-// butterfly's pairing does not change the result
-__device__ VI block_argmax(VI x, VI *sh)
-{
-    int tid = threadIdx.x;
-    x = vi_step<32>(x);
-    x = vi_step<16>(x);
-    x = vi_step<8>(x);
-    x = vi_step<4>(x);
-    x = vi_step<2>(x);
-    x = vi_step<1>(x);
-    if ((tid & 63) == 0) sh[tid >> 6] = x;
-    __syncthreads();
-    VI r = sh[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); w++) r = vi_better(r, sh[w]);
-    __syncthreads();
-    return r;
-}
-
 // v of the lane CTRL names, or v itself where that lane is outside the row
 template <int CTRL>
 __device__ __forceinline__ double dpp_max(double v)
@@ -1780,185 +1761,264 @@ template __global__ void k_hss_colcomp<512, true>(const HssMerge *, const HssNod
 // the ranks, and it is kept: one workgroup walks the tree, and every RRLU step
 // (rrluCauchy, :7-134, rho = 1.02, a swap check every 10 steps) runs across the
 // workgroup's threads, its scalar decisions taken identically by every thread from
-// the same global values.  Statement order is the Fortran's.
+// the same values.  Every element's operations and their order are the Fortran's.
+//
+// The bound is the latency of the pivot steps, one after another on one CU: both sides of
+// a compression sit in LDS (up to C2H_LDS doubles; global scratch beyond), one instance of
+// the step's code serves rows and columns of leaves and parents (eight inlined copies made
+// 69 KB, more than the instruction cache), the next step's searches run inside the update
+// pass, and W, needed only by the swap check and the generator, is formed ten steps at a
+// time with a thread per entry.  n = 2000, leaf 64: 50.7 ms before.
 // ===========================================================================
-#define C2H_WG 1024
+#define C2H_WG 512
+#define C2H_NW (C2H_WG / 64)
+#define C2H_LDS 18432  // doubles of dynamic LDS
 
-// CauchyMax (:166-188): max |u(i) / (D(i) - F)|, i = 1..n, first index
-__device__ VI g_cmax(const double *D, double F, const double *u, int n, VI *red)
+// first largest |U(i) / (X(i) - y)| over i = k .. n (index i - k + 1), i from i0 by step
+template <class DP>
+__device__ __forceinline__ VI c2h_max(DP X, DP U, double y, int k, int n, int i0, int step)
 {
     VI x = {0.0, 0};
-    for (int i = 1 + threadIdx.x; i <= n; i += C2H_WG) x = vi_better(x, VI{fabs(A1(u, i) / (A1(D, i) - F)), i});
-    return block_argmax(x, red);
+    for (int i = k + i0; i <= n; i += step) x = vi_better(x, VI{fabs(A1(U, i) / (A1(X, i) - y)), i - k + 1});
+    return x;
 }
 
-__device__ __forceinline__ void g_dswp(double *a, int i, int j) { double t = A1(a, i); A1(a, i) = A1(a, j); A1(a, j) = t; }
-__device__ __forceinline__ void g_iswp(int *a, int i, int j) { int t = A1(a, i); A1(a, i) = A1(a, j); A1(a, j) = t; }
-
-// CauchyPivtG (:191-243): rook pivoting on the k-th Schur complement
-__device__ void g_pivt(double *D, double *F, double *u, double *v, int *PL, int *PU, int k, double *A, int M, int N,
-                       VI *red)
+// rrluCauchy (:7-134) of the M x N matrix A(i) V(j) / (X(i) - Y(j)) with the pivoting of
+// CauchyPivtG (:191-243) and CauchyPivtG_CP (:246-296); returns Rk.  U: the row generators
+// of the Schur complement, W: those of the interpolation; T1, T2: M scratch each.
+template <class DP, class IP>
+__device__ __forceinline__ int c2h_rrlu(DP X, DP A, DP U, DP W, DP T1, DP T2, IP PL, DP Y, DP V, double tol, int M, int N,
+                                     VI *red, int *s_ii, int *s_nsw)
 {
-    const VI L = g_cmax(D + k - 1, A1(F, k), u + k - 1, M - k + 1, red);
-    const VI R = g_cmax(F + k - 1, A1(D, k), v + k - 1, N - k + 1, red);
-    const double junkL = L.v * fabs(A1(v, k)), junkU = R.v * fabs(A1(u, k));
-    const double piv = fabs(A1(u, k) * A1(v, k) / (A1(D, k) - A1(F, k)));
-    if (junkL <= piv && junkU <= piv) return;
-    int flg = (junkL > junkU) ? 1 : 0, jjL = L.i, jjU = R.i;
-    // every round moves a strictly larger entry into the pivot, so finite data ends
-    // within M + N rounds; the bound only guarantees an exit for overflowed generators
-    for (int round = 0; round < M + N + 2; round++) {
-        if (flg == 1) {
-            const int jj = jjL + k - 1;
-            __syncthreads();  // every wave has read the pivot entries it decided on
-            if (threadIdx.x == 0) { g_dswp(D, k, jj); g_dswp(u, k, jj); g_dswp(A, k, jj); g_iswp(PL, k, jj); }
-            __syncthreads();
-            jjU = g_cmax(F + k - 1, A1(D, k), v + k - 1, N - k + 1, red).i;
-            if (jjU == 1) return;
-            flg = 0;
-        }
-        const int jj = jjU + k - 1;
-        __syncthreads();
-        if (threadIdx.x == 0) { g_dswp(F, k, jj); g_dswp(v, k, jj); g_iswp(PU, k, jj); }
-        __syncthreads();
-        jjL = g_cmax(D + k - 1, A1(F, k), u + k - 1, M - k + 1, red).i;
-        if (jjL == 1) return;
-        flg = 1;
-    }
-}
-
-// CauchyPivtG_CP (:246-296): complete pivoting, one thread per column
-__device__ void g_pivt_cp(double *D, double *F, double *u, double *v, int *PL, int *PU, int k, double *A, int M,
-                          int N, VI *red, int *s_ii)
-{
-    VI best = {0.0, 0};
-    int bestrow = 1;
-    for (int j = 1 + threadIdx.x; j <= N - k + 1; j += C2H_WG) {
-        const double fj = A1(F, k + j - 1);
-        double mv = 0.0;
-        int mi = 1;
-        for (int i = 1; i <= M - k + 1; i++) {
-            const double x = fabs(A1(u, k + i - 1) / (A1(D, k + i - 1) - fj));
-            if (i == 1 || x > mv) { mv = x; mi = i; }
-        }
-        const VI c = {fabs(mv * A1(v, k + j - 1)), j};
-        const VI nb = vi_better(best, c);
-        if (nb.i == c.i) bestrow = mi;
-        best = nb;
-    }
-    const VI win = block_argmax(best, red);
-    if (best.i == win.i && win.i > 0) *s_ii = bestrow;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int ii = *s_ii + k - 1, jj = win.i + k - 1;
-        g_dswp(D, k, ii); g_dswp(u, k, ii); g_dswp(A, k, ii); g_iswp(PL, k, ii);
-        g_dswp(F, k, jj); g_dswp(v, k, jj); g_iswp(PU, k, jj);
-    }
-    __syncthreads();
-}
-
-// rrluCauchy (:7-134) of the M x N matrix A(i) V(j) / (D(i) - F(j)); returns Rk
-__device__ int g_rrlu(double *D, double *F, double *A, double *V, double tol, double *U, double *W, int *PL, int *PU,
-                      int M, int N, VI *red, int *s_ii, unsigned long long &nsw)
-{
-    const int tid = threadIdx.x, mn = M < N ? M : N;
+    const int tid = threadIdx.x, lane = tid & 63, mn = M < N ? M : N;
     const double rho = 1.02;
+    int tog = 0;
     for (int j = 1 + tid; j <= M; j += C2H_WG) { A1(U, j) = A1(A, j); A1(PL, j) = j; }
-    for (int j = 1 + tid; j <= N; j += C2H_WG) A1(PU, j) = j;
     __syncthreads();
-    int Rk = mn;
-    double amax = 0.0;
-    for (int k = 1; k <= mn; k++) {
-        g_pivt(D, F, U, V, PL, PU, k, A, M, N, red);
+    auto swapr = [&](int a, int b) {
+        const double xa = A1(X, a), xb = A1(X, b), ua = A1(U, a), ub = A1(U, b), aa = A1(A, a), ab = A1(A, b);
+        const int pa = A1(PL, a), pb = A1(PL, b);
+        A1(X, a) = xb; A1(X, b) = xa;
+        A1(U, a) = ub; A1(U, b) = ua;
+        A1(A, a) = ab; A1(A, b) = aa;
+        A1(PL, a) = pb; A1(PL, b) = pa;
+    };
+    auto swapc = [&](int a, int b) {
+        const double ya = A1(Y, a), yb = A1(Y, b), va = A1(V, a), vb = A1(V, b);
+        A1(Y, a) = yb; A1(Y, b) = ya;
+        A1(V, a) = vb; A1(V, b) = va;
+    };
+    // W of steps 1 .. K from that of steps 1 .. k0: step q multiplies W(j), j < q, by
+    // (Y(q) - X(j)) / (X(q) - X(j)) and sets W(q) = (X(q) - Y(q)) / A(q) times, then over,
+    // (Y(j) - X(q)), (X(j) - X(q)) for j = 1 .. q - 1.  Positions 1 .. q of X, Y and A do not
+    // change between step q and the next swap check, so ten steps' factors come at once.
+    auto wsteps = [&](int k0, int K) {
+        for (int j = 1 + tid; j <= K; j += C2H_WG) {
+            const double xj = A1(X, j);
+            double w;
+            if (j > k0) {
+                w = (xj - A1(Y, j)) / A1(A, j);
+                for (int q = 1; q < j; q++) w = w * (A1(Y, q) - xj) / (A1(X, q) - xj);
+            } else {
+                w = A1(W, j);
+            }
+            for (int q = (j > k0 ? j : k0) + 1; q <= K; q++) w = w * ((A1(Y, q) - xj) / (A1(X, q) - xj));
+            A1(W, j) = w;
+        }
         __syncthreads();
-        double ukk = A1(U, k) * A1(V, k) / (A1(D, k) - A1(F, k));
+    };
+    int Rk = mn, kw = 0;  // kw: steps W holds
+    double amax = 0.0;
+    bool pre = false;     // pre_l, pre_u hold this step's first searches
+    VI pre_l = {0.0, 0}, pre_u = {0.0, 0};
+    for (int k = 1; k <= mn; k++) {
+        VI L, R;
+        if (pre) {
+            L = pre_l;
+            R = pre_u;
+        } else {
+            L = c2h_max(X, U, A1(Y, k), k, M, tid, C2H_WG);
+            R = c2h_max(Y, V, A1(X, k), k, N, tid, C2H_WG);
+            block_argmax2_t<C2H_NW>(L, R, red, tog);
+        }
+        const double junkL = L.v * fabs(A1(V, k)), junkU = R.v * fabs(A1(U, k));
+        const double piv = fabs(A1(U, k) * A1(V, k) / (A1(X, k) - A1(Y, k)));
+        if (!(junkL <= piv && junkU <= piv)) {
+            int flg = (junkL > junkU) ? 1 : 0, jjL = L.i, jjU = R.i;
+            // a row swap is made after the column search it feeds and its barrier; a column
+            // swap first waits until every thread has read position k
+            if (flg == 0) __syncthreads();
+            // every round moves a strictly larger entry into the pivot, so finite data ends
+            // within M + N rounds; the bound only guarantees an exit for overflowed generators
+            for (int round = 0; round < M + N + 2; round++) {
+                if (flg == 1) {
+                    const int jr = jjL + k - 1;
+                    jjU = block_argmax_t<C2H_NW>(c2h_max(Y, V, A1(X, jr), k, N, tid, C2H_WG), red, tog).i;
+                    if (tid == 0) swapr(k, jr);
+                    if (jjU == 1) break;
+                }
+                if (tid == 0) swapc(k, jjU + k - 1);
+                __syncthreads();
+                // a few hundred rows: every wavefront searches them by itself
+                if (M - k < 256) jjL = wave_argmax<64>(c2h_max(X, U, A1(Y, k), k, M, lane, 64)).i;
+                else jjL = block_argmax_t<C2H_NW>(c2h_max(X, U, A1(Y, k), k, M, tid, C2H_WG), red, tog).i;
+                if (jjL == 1) break;
+                flg = 1;
+            }
+            __syncthreads();
+        }
+        double ukk = A1(U, k) * A1(V, k) / (A1(X, k) - A1(Y, k));
         amax = fmax(amax, fabs(ukk));
         if (fabs(ukk) < tol * amax) {
-            g_pivt_cp(D, F, U, V, PL, PU, k, A, M, N, red, s_ii);
-            ukk = A1(U, k) * A1(V, k) / (A1(D, k) - A1(F, k));
+            // complete pivoting over the Schur complement
+            VI best = {0.0, 0};
+            int bestrow = 1;
+            for (int j = k + tid; j <= N; j += C2H_WG) {
+                const double yj = A1(Y, j);
+                double mv = 0.0;
+                int mi = 0;
+                for (int i = k; i <= M; i++) {
+                    const double u = A1(U, i), den = A1(X, i) - yj;
+                    if (mi != 0 && !may_exceed(u, den, mv)) continue;
+                    const double x = fabs(u / den);
+                    if (mi == 0 || x > mv) { mv = x; mi = i - k + 1; }
+                }
+                const VI c = {fabs(mv * A1(V, j)), j - k + 1};
+                const VI nb = vi_better(best, c);
+                if (nb.i == c.i) bestrow = mi;
+                best = nb;
+            }
+            const VI win = block_argmax_t<C2H_NW>(best, red, tog);
+            if (best.i == win.i && win.i > 0) *s_ii = bestrow;
+            __syncthreads();
+            if (tid == 0) {
+                swapr(k, *s_ii + k - 1);
+                swapc(k, win.i + k - 1);
+            }
+            __syncthreads();
+            ukk = A1(U, k) * A1(V, k) / (A1(X, k) - A1(Y, k));
             amax = fmax(amax, fabs(ukk));
             if (fabs(ukk) < tol * amax) { Rk = k - 1; break; }
         }
-        const double Dk = A1(D, k), Fk = A1(F, k);
-        for (int j = k + 1 + tid; j <= M; j += C2H_WG) A1(U, j) = A1(U, j) * (A1(D, j) - Dk) / (A1(D, j) - Fk);
-        for (int j = k + 1 + tid; j <= N; j += C2H_WG) A1(V, j) = A1(V, j) * (A1(F, j) - Fk) / (A1(F, j) - Dk);
-        for (int j = 1 + tid; j <= k - 1; j += C2H_WG) A1(W, j) = A1(W, j) * ((Fk - A1(D, j)) / (Dk - A1(D, j)));
-        __syncthreads();
-        if (tid == 0) {
-            double wk = (Dk - Fk) / A1(A, k);
-            for (int j = 1; j <= k - 1; j++) wk = wk * (A1(F, j) - Dk) / (A1(D, j) - Dk);
-            A1(W, k) = wk;
+        // generators of the next Schur complement; unless a swap check follows, the next
+        // step's first searches run inside the passes
+        const double Xk = A1(X, k), Yk = A1(Y, k);
+        const bool fuse = k + 1 <= mn && k % 10 != 0;
+        const double Xn = fuse ? A1(X, k + 1) : 0.0, Yn = fuse ? A1(Y, k + 1) : 0.0;
+        VI x1 = {0.0, 0}, y1 = {0.0, 0};
+        for (int j = k + 1 + tid; j <= M; j += C2H_WG) {
+            const double xj = A1(X, j), u = A1(U, j) * (xj - Xk) / (xj - Yk);
+            A1(U, j) = u;
+            if (fuse) x1 = vi_better(x1, VI{fabs(u / (xj - Yn)), j - k});
         }
-        __syncthreads();
+        for (int j = k + 1 + tid; j <= N; j += 2 * C2H_WG) {
+            const int j2 = j + C2H_WG;
+            const double ya = A1(Y, j), va = A1(V, j), yb = A1(Y, min(j2, N)), vb = A1(V, min(j2, N));
+            const double na = va * (ya - Yk) / (ya - Xk), nb = vb * (yb - Yk) / (yb - Xk);
+            A1(V, j) = na;
+            if (j2 <= N) A1(V, j2) = nb;
+            if (fuse) {
+                y1 = vi_better(y1, VI{fabs(na / (ya - Xn)), j - k});
+                if (j2 <= N) y1 = vi_better(y1, VI{fabs(nb / (yb - Xn)), j2 - k});
+            }
+        }
+        pre = fuse;
+        if (fuse) {
+            block_argmax2_t<C2H_NW>(x1, y1, red, tog);
+            pre_l = x1;
+            pre_u = y1;
+        } else {
+            __syncthreads();
+        }
         if (k % 10 != 0) continue;
+        wsteps(kw, k);
+        kw = k;
         // each swap raises |det| of the pivot block by more than rho; bounded all the same
         for (int sw = 0; sw < 2 * M + 8; sw++) {
-            // searchMax2 (:137-163): the largest entry of Mat_N(i, j) = U(k+i) W(j) / (D(k+i) - D(j))
+            // searchMax2 (:137-163): the largest entry of Mat_N(i, j) = U(k+i) W(j) / (X(k+i) - X(j)),
+            // G lanes to a column
             VI x = {0.0, 0};
             int xrow = 1;
-            for (int jc = 1 + tid; jc <= k; jc += C2H_WG) {
-                const double dj = A1(D, jc);
-                double mv = 0.0;
-                int mi = 1;
-                for (int i = 1; i <= M - k; i++) {
-                    const double t = fabs(A1(U, k + i) / (A1(D, k + i) - dj));
-                    if (i == 1 || t > mv) { mv = t; mi = i; }
+            const int G = scan_lanes(k, C2H_WG), g = tid & (G - 1);
+            for (int jc = 1 + tid / G; jc - tid / G <= k; jc += C2H_WG / G) {
+                VI e = {0.0, 0};
+                if (jc <= k) {
+                    const double xj = A1(X, jc);
+                    for (int i = 1 + g; i <= M - k; i += G)
+                        e = vi_better(e, VI{fabs(A1(U, k + i) / (A1(X, k + i) - xj)), i});
                 }
-                const VI c = {mv * fabs(A1(W, jc)), jc};
-                const VI nb = vi_better(x, c);
-                if (nb.i == c.i) xrow = mi;
-                x = nb;
+                e = group_argmax(e, G);
+                if (jc <= k) {
+                    const VI c = {e.v * fabs(A1(W, jc)), jc};
+                    const VI nb = vi_better(x, c);
+                    if (nb.i == c.i) xrow = e.i > 0 ? e.i : 1;
+                    x = nb;
+                }
             }
-            const VI win = block_argmax(x, red);
-            if (x.i == win.i && win.i > 0) *s_ii = xrow;
-            __syncthreads();
+            const VI win = block_argmax_t<C2H_NW>(x, red, tog);
             if (!(win.v > rho)) break;
-            nsw++;
+            if (x.i == win.i && g == 0) *s_ii = xrow;
+            __syncthreads();
             const int ii = win.i, jj = *s_ii + k;
-            const double Dii = A1(D, ii), Djj = A1(D, jj);
-            for (int j = k + 1 + tid; j <= N; j += C2H_WG) A1(V, j) = A1(V, j) * ((A1(F, j) - Dii) / (A1(F, j) - Djj));
+            const double Dii = A1(X, ii), Djj = A1(X, jj);
+            for (int j = k + 1 + tid; j <= N; j += C2H_WG) A1(V, j) = A1(V, j) * ((A1(Y, j) - Dii) / (A1(Y, j) - Djj));
             for (int j = k + 1 + tid; j <= M; j += C2H_WG)
-                if (j != jj) A1(U, j) = A1(U, j) * ((A1(D, j) - Djj) / (A1(D, j) - Dii));
-            for (int j = 1 + tid; j <= k; j += C2H_WG)
-                if (j != ii) A1(W, j) = A1(W, j) * ((A1(D, j) - Dii) / (A1(D, j) - Djj));
+                if (j != jj) A1(U, j) = A1(U, j) * ((A1(X, j) - Djj) / (A1(X, j) - Dii));
+            for (int j = 1 + tid; j <= k; j += C2H_WG) {
+                const double xj = A1(X, j), yj = A1(Y, j);
+                if (j != ii) A1(W, j) = A1(W, j) * ((xj - Dii) / (xj - Djj));
+                // the factors of U(jj) and W(ii); 1 at j = ii leaves the products' bits
+                A1(T1, j) = j == ii ? 1.0 : (Dii - xj) / (Dii - yj);
+                A1(T2, j) = j == ii ? 1.0 : (yj - Djj) / (xj - Djj);
+            }
             __syncthreads();
             if (tid == 0) {
-                double uj = A1(A, ii) * ((Dii - Djj) / (Dii - A1(F, ii)));
-                double wi = (Djj - A1(F, ii)) / A1(A, jj);
+                const double yii = A1(Y, ii);
+                double uj = A1(A, ii) * ((Dii - Djj) / (Dii - yii));
+                double wi = (Djj - yii) / A1(A, jj);
                 for (int j = 1; j <= k; j++) {
-                    if (j == ii) continue;
-                    uj = uj * ((Dii - A1(D, j)) / (Dii - A1(F, j)));
-                    wi = wi * ((A1(F, j) - Djj) / (A1(D, j) - Djj));
+                    uj = uj * A1(T1, j);
+                    wi = wi * A1(T2, j);
                 }
+                const double xi = A1(X, ii), xj = A1(X, jj), ai = A1(A, ii), aj = A1(A, jj);
+                const int pi = A1(PL, ii), pj = A1(PL, jj);
                 A1(U, jj) = uj;
                 A1(W, ii) = wi;
-                g_iswp(PL, ii, jj);
-                g_dswp(D, ii, jj);
-                g_dswp(A, ii, jj);
+                A1(PL, ii) = pj; A1(PL, jj) = pi;
+                A1(X, ii) = xj; A1(X, jj) = xi;
+                A1(A, ii) = aj; A1(A, jj) = ai;
+                *s_nsw += 1;
             }
             __syncthreads();
         }
     }
-    __syncthreads();
+    wsteps(kw, Rk);
     return Rk;
 }
 
-// comprcauchy (:616-725): rows ('r': M node rows against N outside columns) or
-// columns ('c': M node columns against N outside rows) of node `nodi`; the
-// interpolative generator (Cauchylike2, :743-778, rows or columns put back in the
-// node's order) goes to the arena
-__device__ int g_compr(const C2H &C, bool row, double *D, double *F, double *U, double *V, int M, int N, int nodi,
-                       VI *red, int *s_ii, long &top, unsigned long long &nsw)
+// comprcauchy (:616-725) of one side of node `nodi` ('r': M node rows against N outside
+// columns, 'c': M node columns against N outside rows): gathers the node's side from
+// (A, Au) at m0 and the outside from (B, Bv) -- the stacked skeletons 1 .. cs - 1, then the
+// originals after `last` --, runs the RRLU, writes the interpolative generator
+// (Cauchylike2, :743-778, in the node's order) to the arena and the skeleton back to
+// (A, Au) at o0.  The six node arrays lie st apart at w.  Returns its rank, -1 when the arena is full.
+template <class DP, class IP>
+__device__ __forceinline__ int c2h_compr(const C2H &C, bool row, DP w, long st, IP PL, IP inv, DP Y, DP V, int m0, int M, int cs,
+                                         int last, int N, int o0, int nodi, long &top, VI *red, int *s_ii, int *s_nsw)
 {
-    const int tid = threadIdx.x, mn = M < N ? M : N;
-    for (int j = 1 + tid; j <= M; j += C2H_WG) A1(C.Z, j) = 0.0;
-    for (int j = 1 + tid; j <= mn; j += C2H_WG) A1(C.W, j) = 0.0;
+    const int tid = threadIdx.x;
+    DP X = w, A = w + st, U = w + 2 * st, W = w + 3 * st, T1 = w + 4 * st, T2 = w + 5 * st;
+    double *Ag = row ? C.D : C.F, *Aug = row ? C.U : C.V, *Bg = row ? C.F : C.D, *Bvg = row ? C.V : C.U;
+    for (int j = tid; j < M; j += C2H_WG) { X[j] = A1(Ag, m0 + j); A[j] = A1(Aug, m0 + j); W[j] = 0.0; }
+    for (int j = tid; j < N; j += C2H_WG) {
+        const int src = (j < cs - 1) ? j + 1 : last + 1 + (j - (cs - 1));
+        Y[j] = A1(Bg, src);
+        V[j] = A1(Bvg, src);
+    }
     __syncthreads();
-    const int Rk = row ? g_rrlu(D, F, U, V, C.tol, C.Z, C.W, C.PL, C.PU, M, N, red, s_ii, nsw)
-                       : g_rrlu(F, D, V, U, C.tol, C.Z, C.W, C.PL, C.PU, M, N, red, s_ii, nsw);
-    const double *X = row ? D : F;
-    // invp: PU (free after the RRLU) takes the position of every original index
-    for (int i = 1 + tid; i <= M; i += C2H_WG) A1(C.PU, A1(C.PL, i)) = i;
+    const int Rk = c2h_rrlu<DP, IP>(X, A, U, W, T1, T2, PL, Y, V, C.tol, M, N, red, s_ii, s_nsw);
+    // inverse of the row permutation
+    for (int i = 1 + tid; i <= M; i += C2H_WG) A1(inv, A1(PL, i)) = i;
     const int r = Rk < M ? Rk : M;
     const long off = top;
     __syncthreads();
@@ -1967,28 +2027,21 @@ __device__ int g_compr(const C2H &C, bool row, double *D, double *F, double *U, 
         return -1;
     }
     double *Q = C.arena + off;
-    if (row) {
-        for (long e = tid; e < (long)M * r; e += C2H_WG) {
-            const int i = (int)(e % M) + 1, j = (int)(e / M) + 1, s = A1(C.PU, i);
-            double q;
-            if (Rk >= M) q = (s == j) ? 1.0 : 0.0;
-            else if (s <= r) q = (s == j) ? 1.0 : 0.0;
-            else q = A1(C.Z, s) * A1(C.W, j) / (A1(X, s) - A1(X, j));
-            Q[e] = q;
-        }
-        if (tid == 0) { C.usz[2 * (nodi - 1)] = M; C.usz[2 * (nodi - 1) + 1] = r; C.pu[nodi - 1] = off; }
-    } else {
-        for (long e = tid; e < (long)M * r; e += C2H_WG) {
-            const int i = (int)(e % r) + 1, j = (int)(e / r) + 1, s = A1(C.PU, j);
-            double q;
-            if (Rk >= M) q = (s == i) ? 1.0 : 0.0;
-            else if (s <= r) q = (s == i) ? 1.0 : 0.0;
-            else q = A1(C.W, i) * A1(C.Z, s) / (A1(X, s) - A1(X, i));
-            Q[e] = q;
-        }
-        if (tid == 0) { C.vsz[2 * (nodi - 1)] = r; C.vsz[2 * (nodi - 1) + 1] = M; C.pv[nodi - 1] = off; }
+    for (long e = tid; e < (long)M * r; e += C2H_WG) {
+        // rows: Q is M x r, entry (i, j); columns: r x M, entry (i, j) of the transpose
+        const int a = (int)(e % (row ? M : r)) + 1, b = (int)(e / (row ? M : r)) + 1;
+        const int i = row ? a : b, j = row ? b : a, s = A1(inv, i);
+        double q;
+        if (Rk >= M || s <= r) q = (s == j) ? 1.0 : 0.0;
+        else q = A1(U, s) * A1(W, j) / (A1(X, s) - A1(X, j));
+        Q[e] = q;
+    }
+    if (tid == 0) {
+        if (row) { C.usz[2 * (nodi - 1)] = M; C.usz[2 * (nodi - 1) + 1] = r; C.pu[nodi - 1] = off; }
+        else { C.vsz[2 * (nodi - 1)] = r; C.vsz[2 * (nodi - 1) + 1] = M; C.pv[nodi - 1] = off; }
     }
     top = off + (long)M * r;
+    for (int j = tid; j < Rk; j += C2H_WG) { A1(Ag, o0 + j) = X[j]; A1(Aug, o0 + j) = A[j]; }
     __syncthreads();
     return Rk;
 }
@@ -2003,99 +2056,64 @@ __device__ void g_cfill(double *a, int lda, const double *D, const double *F, co
     }
 }
 
-__global__ __launch_bounds__(C2H_WG) void k_cauchy2hss(C2H C)
+__global__ __launch_bounds__(C2H_WG) void k_cauchy2hss(C2H C, int lds_cap)
 {
-    __shared__ VI red[C2H_WG / 64];
-    __shared__ int s_ii;
+    extern __shared__ double hss_dyn[];  // lds_cap doubles
+    __shared__ VI red[4 * C2H_NW];
+    __shared__ int s_ii, s_nsw;
+    typedef __attribute__((address_space(3))) int lint;
     const int tid = threadIdx.x, lda = C.n;
     long top = 0;               // arena bump, the same in every thread
-    unsigned long long nsw = 0;
     int ns = 1;
     int *lsr = C.lsr, *lsc = C.lsc;
-    if (tid == 0) { A1(lsr, 1) = 1; A1(lsc, 1) = 1; }
+    if (tid == 0) { A1(lsr, 1) = 1; A1(lsc, 1) = 1; s_nsw = 0; }
     __syncthreads();
-    // gather the node's row side (D, U at idx(j)) and the outside column side
-    // (the stacked column skeletons 1..cs-1, then the original columns after `last`)
-    auto gather = [&](bool row, int m0, int mi, int cs, int last, int nt) {
-        double *A = row ? C.D : C.F, *Au = row ? C.U : C.V, *B = row ? C.F : C.D, *Bv = row ? C.V : C.U;
-        double *Ai = row ? C.Di : C.Fi, *Aui = row ? C.Ui : C.Vi, *Bi = row ? C.Fi : C.Di, *Bvi = row ? C.Vi : C.Ui;
-        for (int j = tid; j < mi; j += C2H_WG) { Ai[j] = A1(A, m0 + j); Aui[j] = A1(Au, m0 + j); }
-        for (int j = tid; j < nt; j += C2H_WG) {
-            const int src = (j < cs - 1) ? j + 1 : last + 1 + (j - (cs - 1));
-            Bi[j] = A1(B, src);
-            Bvi[j] = A1(Bv, src);
-        }
-        __syncthreads();
-    };
     for (int i = 1; i <= C.ltr; i++) {
         const int c1 = C.ch[2 * (i - 1)], c2 = C.ch[2 * (i - 1) + 1];
         const int l1 = C.rng[2 * (i - 1)], l2 = C.rng[2 * (i - 1) + 1];
-        if (c1 == 0) {  // leaf
-            const int mi = l2 - l1 + 1, nii = lda - l2;
+        const bool leaf = c1 == 0;
+        if (leaf) {
+            const int mi = l2 - l1 + 1;
             g_cfill(C.dd + C.pd[i - 1], mi, C.D + l1 - 1, C.F + l1 - 1, C.U + l1 - 1, C.V + l1 - 1, mi, mi);
             if (tid == 0) C.dsz[i - 1] = mi;
-            int cs = (ns == 1) ? 1 : A1(lsc, ns);
-            gather(true, l1, mi, cs, l2, nii + cs - 1);
-            int Rk = g_compr(C, true, C.Di, C.Fi, C.Ui, C.Vi, mi, nii + cs - 1, i, red, &s_ii, top, nsw);
-            if (Rk < 0) return;
-            const int r0 = A1(lsr, ns);
-            for (int j = tid; j < Rk; j += C2H_WG) { A1(C.D, r0 + j) = C.Di[j]; A1(C.U, r0 + j) = C.Ui[j]; }
-            __syncthreads();
-            if (tid == 0) A1(lsr, ns + 1) = r0 + Rk;
-            __syncthreads();
-            const int rs = (ns == 1) ? 1 : A1(lsr, ns);
-            gather(false, l1, mi, rs, l2, nii + rs - 1);
-            Rk = g_compr(C, false, C.Di, C.Fi, C.Ui, C.Vi, mi, nii + rs - 1, i, red, &s_ii, top, nsw);
-            if (Rk < 0) return;
-            const int q0 = A1(lsc, ns);
-            for (int j = tid; j < Rk; j += C2H_WG) { A1(C.F, q0 + j) = C.Fi[j]; A1(C.V, q0 + j) = C.Vi[j]; }
-            __syncthreads();
-            if (tid == 0) A1(lsc, ns + 1) = q0 + Rk;
-            __syncthreads();
-            ns++;
         } else {  // parent: B of both children, then its own compressions
-            int mi = A1(lsr, ns - 1) - A1(lsr, ns - 2), nii = A1(lsc, ns) - A1(lsc, ns - 1);
-            if (top + (long)mi * nii > C.arena_cap) { if (tid == 0) atomicOr(C.err, 2); return; }
-            g_cfill(C.arena + top, mi, C.D + A1(lsr, ns - 2) - 1, C.F + A1(lsc, ns - 1) - 1, C.U + A1(lsr, ns - 2) - 1,
-                    C.V + A1(lsc, ns - 1) - 1, mi, nii);
-            if (tid == 0) { C.bsz[2 * (c1 - 1)] = mi; C.bsz[2 * (c1 - 1) + 1] = nii; C.pb[c1 - 1] = top; }
-            top += (long)mi * nii;
-            mi = A1(lsr, ns) - A1(lsr, ns - 1);
-            nii = A1(lsc, ns - 1) - A1(lsc, ns - 2);
-            if (top + (long)mi * nii > C.arena_cap) { if (tid == 0) atomicOr(C.err, 2); return; }
-            g_cfill(C.arena + top, mi, C.D + A1(lsr, ns - 1) - 1, C.F + A1(lsc, ns - 2) - 1, C.U + A1(lsr, ns - 1) - 1,
-                    C.V + A1(lsc, ns - 2) - 1, mi, nii);
-            if (tid == 0) { C.bsz[2 * (c2 - 1)] = mi; C.bsz[2 * (c2 - 1) + 1] = nii; C.pb[c2 - 1] = top; }
-            top += (long)mi * nii;
-            __syncthreads();
+            for (int t = 0; t < 2; t++) {
+                const int cr = t ? ns - 1 : ns - 2, cc = t ? ns - 2 : ns - 1, cnode = t ? c2 : c1;
+                const int r0 = A1(lsr, cr), mi = A1(lsr, cr + 1) - r0, q0 = A1(lsc, cc), ni = A1(lsc, cc + 1) - q0;
+                if (top + (long)mi * ni > C.arena_cap) { if (tid == 0) atomicOr(C.err, 2); return; }
+                g_cfill(C.arena + top, mi, C.D + r0 - 1, C.F + q0 - 1, C.U + r0 - 1, C.V + q0 - 1, mi, ni);
+                if (tid == 0) { C.bsz[2 * (cnode - 1)] = mi; C.bsz[2 * (cnode - 1) + 1] = ni; C.pb[cnode - 1] = top; }
+                top += (long)mi * ni;
+            }
             if (i == C.ltr) break;
-            // rows of the merged skeleton against the stacked columns before and the columns after
-            mi = A1(lsr, ns) - A1(lsr, ns - 2);
-            nii = lda - l2;
-            int cs = (ns == 3) ? 1 : A1(lsc, ns - 2);
-            gather(true, A1(lsr, ns - 2), mi, cs, l2, nii + cs - 1);
-            int Rk = g_compr(C, true, C.Di, C.Fi, C.Ui, C.Vi, mi, nii + cs - 1, i, red, &s_ii, top, nsw);
-            if (Rk < 0) return;
-            const int r0 = A1(lsr, ns - 2);
-            for (int j = tid; j < Rk; j += C2H_WG) { A1(C.D, r0 + j) = C.Di[j]; A1(C.U, r0 + j) = C.Ui[j]; }
-            __syncthreads();
-            if (tid == 0) A1(lsr, ns - 1) = r0 + Rk;
-            __syncthreads();
-            // columns of the merged skeleton
-            mi = A1(lsc, ns) - A1(lsc, ns - 2);
-            const int rs = (ns == 3) ? 1 : A1(lsr, ns - 2);
-            gather(false, A1(lsc, ns - 2), mi, rs, l2, nii + rs - 1);
-            Rk = g_compr(C, false, C.Di, C.Fi, C.Ui, C.Vi, mi, nii + rs - 1, i, red, &s_ii, top, nsw);
-            if (Rk < 0) return;
-            const int q0 = A1(lsc, ns - 2);
-            for (int j = tid; j < Rk; j += C2H_WG) { A1(C.F, q0 + j) = C.Fi[j]; A1(C.V, q0 + j) = C.Vi[j]; }
-            __syncthreads();
-            if (tid == 0) A1(lsc, ns - 1) = q0 + Rk;
-            __syncthreads();
-            ns--;
         }
+        __syncthreads();
+        // a leaf's rows and columns are the originals l1 .. l2, a parent's the merged
+        // skeletons of its children; the skeletons of the nodes before it and the
+        // originals after it are outside
+        const int base = leaf ? ns : ns - 2;  // stack position this node's skeletons go to
+        for (int side = 0; side < 2; side++) {
+            const bool row = side == 0;
+            const int *own = row ? lsr : lsc, *oth = row ? lsc : lsr;
+            const int m0 = leaf ? l1 : A1(own, base), M = leaf ? l2 - l1 + 1 : A1(own, ns) - A1(own, base);
+            const int cs = base == 1 ? 1 : A1(oth, base), N = lda - l2 + cs - 1, o0 = A1(own, base);
+            __syncthreads();  // every thread has read the stack before it changes
+            int Rk;
+            if (7L * M + 2L * N + 2 <= lds_cap) {
+                ldbl *w = (ldbl *)hss_dyn;
+                Rk = c2h_compr<ldbl *, lint *>(C, row, w, (long)M, (lint *)(w + 6 * M), (lint *)(w + 6 * M) + M, w + 7 * M,
+                                               w + 7 * M + N, m0, M, cs, l2, N, o0, i, top, red, &s_ii, &s_nsw);
+            } else {
+                Rk = c2h_compr<gdblw *, gint *>(C, row, (gdblw *)C.S, (long)C.n, (gint *)C.PL, (gint *)C.PU, (gdblw *)C.Fi,
+                                                (gdblw *)C.Vi, m0, M, cs, l2, N, o0, i, top, red, &s_ii, &s_nsw);
+            }
+            if (Rk < 0) return;
+            if (tid == 0) A1(row ? lsr : lsc, base + 1) = o0 + Rk;
+            __syncthreads();
+        }
+        ns = base + 1;
     }
-    if (tid == 0) *C.nswap = nsw;
+    if (tid == 0) *C.nswap = (unsigned long long)s_nsw;
 }
 
 // the dense general Cauchy-like matrix (fallback for a tree of one leaf)
