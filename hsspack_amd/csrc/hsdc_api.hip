@@ -66,6 +66,7 @@ struct M2hJob {
     int w, m;
     long toff;
     long boff;
+    int lq;
 };
 struct M2hBlk {
     int start, count;
@@ -81,6 +82,11 @@ __global__ void k_m2h_gather(const M2hJob *, const double *, long, double *);
 #define M2H_SVD_WG 1024     // threads per block of k_m2h_svd
 #define M2H_LDS 19800       // LDS doubles it may take (160 KB less its static arrays)
 __global__ void k_m2h_svd(const M2hJob *, double *, double *, double, int *, int *, int);
+struct M2hChunk { long src, dst; int rows, m, lds, ldd; };
+__global__ void k_m2h_qr(const M2hChunk *, double *);
+// rows of an m-column matrix that one workgroup reduces in LDS (0: more columns than the
+// tree reduction takes; at least 2 m, so every stage shrinks the matrix)
+static int m2h_qr_rows(int m) { return m < 1 || m > 96 ? 0 : std::min(512, M2H_LDS / m); }
 __global__ void k_m2h_sketch(const M2hJob *, const M2hJob *, const double *, double *, unsigned long long);
 __global__ void k_m2h_rows(const M2hBlk *, int, const M2hJob *, const double *, const double *, long, int, double *,
                            long);
@@ -2811,6 +2817,7 @@ static int mat2hss_build(hsdc_ctx *c, const double *dA, int n, int ni, double to
         std::vector<M2hJob> jobs(2 * nn), sk(2 * nn);
         long so = 0, bo = 0;
         bool any_sketch = false;
+        std::vector<std::vector<M2hChunk>> stages;  // the tree reductions of tall matrices
         for (int q = 0; q < nn; q++) {
             const int nd = nds[q];
             const int f = T.c1[nd] ? T.c1[nd] : nd, l = T.c1[nd] ? T.c2[nd] : nd;
@@ -2829,16 +2836,35 @@ static int mat2hss_build(hsdc_ctx *c, const double *dA, int n, int ni, double to
                 J.w = sd == 0 ? nc - cn : nr - rn;
                 J.toff = so;
                 J.boff = bo;
+                J.lq = 1;
                 bo += (long)J.m * J.m + 2L * J.m;
                 M2hJob &K = sk[2 * q + sd];
                 K = J;
                 if (rsvd && J.w > 50 && J.w > J.m + 10) {  // mat2hssvdr's sampling test
                     K.w = J.m + 10;
+                    K.lq = 0;
                     K.toff = so + (long)J.w * J.m;
                     so += (long)J.w * J.m + (long)K.w * J.m + 2L * J.m * J.m;
                     any_sketch = true;
                 } else {
                     so += (long)J.w * J.m + 2L * J.m * J.m;
+                    // chunks of rows to their R factors, until one workgroup holds what is left;
+                    // the stages alternate between the matrix and a stack behind it
+                    const int cr = m2h_qr_rows(J.m);
+                    const long stack = so;
+                    for (int st = 0; cr > 0 && K.w > cr; st++) {
+                        const int nch = (K.w + cr - 1) / cr;
+                        const long dst = (st & 1) ? J.toff : stack;
+                        if ((int)stages.size() <= st) stages.resize(st + 1);
+                        for (int z = 0, r0 = 0; z < nch; z++) {
+                            const int r1 = (int)((long)K.w * (z + 1) / nch);
+                            stages[st].push_back({K.toff + r0, dst + (long)z * J.m, r1 - r0, J.m, K.w, nch * J.m});
+                            r0 = r1;
+                        }
+                        if (st == 0) so += (long)nch * J.m * J.m;
+                        K.w = nch * J.m;
+                        K.toff = dst;
+                    }
                 }
             }
         }
@@ -2846,10 +2872,16 @@ static int mat2hss_build(hsdc_ctx *c, const double *dA, int n, int ni, double to
         CK(ensure(c->yb, sizeof(double) * (size_t)std::max(bo, 1L)));
         double *S = (double *)c->xb.p, *Bs = (double *)c->yb.p;
         const size_t jb = al64(sizeof(M2hJob) * jobs.size());
-        CK(ensure(c->tabs, 2 * jb + 64 + sizeof(int) * jobs.size()));
+        std::vector<M2hChunk> chunks;
+        for (auto &v : stages) chunks.insert(chunks.end(), v.begin(), v.end());
+        const size_t cbytes = al64(sizeof(M2hChunk) * chunks.size());
+        CK(ensure(c->tabs, 2 * jb + cbytes + 64 + sizeof(int) * jobs.size()));
         char *tb = (char *)c->tabs.p;
         M2hJob *dj = (M2hJob *)tb, *dk = (M2hJob *)(tb + jb);
-        int *derr = (int *)(tb + 2 * jb), *drank = derr + 16;
+        M2hChunk *dc = (M2hChunk *)(tb + 2 * jb);
+        int *derr = (int *)(tb + 2 * jb + cbytes), *drank = derr + 16;
+        if (!chunks.empty())
+            HK(hipMemcpyAsync(dc, chunks.data(), sizeof(M2hChunk) * chunks.size(), hipMemcpyHostToDevice, s));
         HK(hipMemcpyAsync(dj, jobs.data(), sizeof(M2hJob) * jobs.size(), hipMemcpyHostToDevice, s));
         HK(hipMemcpyAsync(dk, sk.data(), sizeof(M2hJob) * sk.size(), hipMemcpyHostToDevice, s));
         HK(hipMemsetAsync(derr, 0, sizeof(int), s));
@@ -2858,8 +2890,18 @@ static int mat2hss_build(hsdc_ctx *c, const double *dA, int n, int ni, double to
         if (any_sketch)
             hipLaunchKernelGGL(k_m2h_sketch, dim3(32, (unsigned)jobs.size()), dim3(WGS), 0, s, (const M2hJob *)dj,
                                (const M2hJob *)dk, (const double *)S, S, seed);
-        long need = 0;  // LDS of the largest side's R and V
-        for (const M2hJob &J : sk) need = std::max(need, (long)J.m * std::min(J.m, J.w) + (J.w >= J.m ? (long)J.m * J.m : 0));
+        for (auto &v : stages) {
+            long need = 0;
+            for (const M2hChunk &C : v) need = std::max(need, (long)C.rows * C.m);
+            hipLaunchKernelGGL(k_m2h_qr, dim3((unsigned)v.size()), dim3(M2H_SVD_WG), sizeof(double) * (size_t)need, s,
+                               (const M2hChunk *)dc, S);
+            dc += v.size();
+        }
+        long need = 0;  // LDS of the largest side's R and V, or of the matrix they come from
+        for (const M2hJob &J : sk) {
+            need = std::max(need, (long)J.m * std::min(J.m, J.w) + (J.w >= J.m ? (long)J.m * J.m : 0));
+            if (J.w <= m2h_qr_rows(J.m)) need = std::max(need, (long)J.w * J.m);
+        }
         const int ldsn = (int)std::min(need, (long)M2H_LDS);
         hipLaunchKernelGGL(k_m2h_svd, dim3((unsigned)jobs.size()), dim3(M2H_SVD_WG), sizeof(double) * (size_t)ldsn, s,
                            (const M2hJob *)dk, S, Bs, tol, drank, derr, ldsn);

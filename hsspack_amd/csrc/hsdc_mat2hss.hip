@@ -45,6 +45,7 @@ struct M2hJob {
     int w, m;            // context length and own length of this side
     long toff;           // T, then R (m x m), V (m x m) at toff + w m, + m m
     long boff;           // basis (m x m) and singular values (m)
+    int lq;              // 1: a second QR before the Jacobi sweeps
 };
 
 // ---------------------------------------------------------------------------
@@ -88,6 +89,7 @@ __global__ __launch_bounds__(MWG) void k_m2h_gather(const M2hJob *jobs, const do
 // 26 ms.
 // ---------------------------------------------------------------------------
 #define M2H_SVD_WG 1024
+#define M2H_QM 100  // columns of a QR in LDS (R and V both fit up to 99)
 
 typedef __attribute__((address_space(3))) double m2h_ldbl;
 typedef __attribute__((address_space(1))) double m2h_gdbl;
@@ -97,49 +99,83 @@ typedef __attribute__((address_space(1))) double m2h_gdbl;
 // Returns false when the sweeps did not converge.
 template <class RP, class VP>
 __device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, double *sv, int *ord, double *B,
-                                           int *s_rot)
+                                           int *s_rot, double *s_part)
 {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, NW = M2H_SVD_WG / 64;
     const int L = m, PP = P + (P & 1);
     bool conv = P < 2;
+    // Columns parallel to the last bit (a block of exact rank one) stay parallel: every
+    // sweep only shrinks the smaller by about eps, and once the squares are denormal the
+    // angles are noise and the sweeps never end.  A column below 2^-300 of the matrix's norm
+    // is left alone.
+    double part = 0.0;
+    for (long e = tid; e < (long)m * P; e += M2H_SVD_WG) part += R[e] * R[e];
+    part = team_bfly(part, 64);
+    if (lane == 0) s_part[wv] = part;
+    __syncthreads();
+    double lim = 0.0;
+    for (int q = 0; q < NW; q++) lim += s_part[q];
+    lim *= 0x1p-600;
     for (int sweep = 0; sweep < 60 && !conv; sweep++) {
         if (tid == 0) *s_rot = 0;
         __syncthreads();
         bool rot = false;
         for (int r = 0; r < PP - 1; r++) {
-            for (int pr = wv; pr < PP / 2; pr += NW) {
-                int a = m2h_rr(pr, r, PP), b = m2h_rr(PP - 1 - pr, r, PP);
-                if (a > b) { const int t = a; a = b; b = t; }
-                if (b >= P) continue;  // uniform over the wavefront
-                const RP ca = R + (long)a * m, cb = R + (long)b * m;
-                double al = 0.0, be = 0.0, ga = 0.0;
-                for (int k = lane; k < L; k += 64) {
-                    const double x = ca[k], y = cb[k];
-                    al += x * x; be += y * y; ga += x * y;
+            // two pairs per wavefront at a time: their sums and rotations overlap
+            for (int pr = wv; pr < PP / 2; pr += 2 * NW) {
+                int pa[2], pb[2];
+                bool ok[2];
+                double al[2] = {0.0, 0.0}, be[2] = {0.0, 0.0}, ga[2] = {0.0, 0.0}, cc[2], ss[2];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int q = pr + u * NW;
+                    const int x = m2h_rr(q, r, PP), y = m2h_rr(PP - 1 - q, r, PP);
+                    pa[u] = x < y ? x : y;
+                    pb[u] = x < y ? y : x;
+                    ok[u] = q < PP / 2 && pb[u] < P;  // uniform over the wavefront
                 }
-                al = team_bfly(al, 64); be = team_bfly(be, 64); ga = team_bfly(ga, 64);
-                if (ga == 0.0 || !(fabs(ga) > L * HSDC_EPS * sqrt(al * be))) continue;
-                const double ze = (be - al) / (2.0 * ga);
-                const double t = (ze >= 0.0 ? 1.0 : -1.0) / (fabs(ze) + sqrt(1.0 + ze * ze));
-                const double cc = 1.0 / sqrt(1.0 + t * t), ss = cc * t;
-                // columns parallel to the last bit (a block of exact rank one): every sweep
-                // shrinks the smaller one by about eps until its square underflows and the
-                // angle vanishes; a rotation that changes nothing is not counted
-                if (ss == 0.0) continue;
-                for (int k = lane; k < L; k += 64) {
-                    const double x = ca[k], y = cb[k];
-                    ca[k] = cc * x - ss * y;
-                    cb[k] = ss * x + cc * y;
-                }
-                if (qr) {
-                    const VP va = V + (long)a * m, vb = V + (long)b * m;
-                    for (int k = lane; k < m; k += 64) {
-                        const double x = va[k], y = vb[k];
-                        va[k] = cc * x - ss * y;
-                        vb[k] = ss * x + cc * y;
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    if (!ok[u]) continue;
+                    const RP ca = R + (long)pa[u] * m, cb = R + (long)pb[u] * m;
+                    for (int k = lane; k < L; k += 64) {
+                        const double x = ca[k], y = cb[k];
+                        al[u] += x * x; be[u] += y * y; ga[u] += x * y;
                     }
                 }
-                rot = true;
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    al[u] = team_bfly(al[u], 64); be[u] = team_bfly(be[u], 64); ga[u] = team_bfly(ga[u], 64);
+                }
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    if (ga[u] == 0.0 || fmin(al[u], be[u]) <= lim ||
+                        !(fabs(ga[u]) > L * HSDC_EPS * sqrt(al[u] * be[u])))
+                        ok[u] = false;
+                    const double ze = (be[u] - al[u]) / (2.0 * ga[u]);
+                    const double t = (ze >= 0.0 ? 1.0 : -1.0) / (fabs(ze) + sqrt(1.0 + ze * ze));
+                    cc[u] = 1.0 / sqrt(1.0 + t * t);
+                    ss[u] = cc[u] * t;
+                }
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    if (!ok[u]) continue;
+                    const RP ca = R + (long)pa[u] * m, cb = R + (long)pb[u] * m;
+                    for (int k = lane; k < L; k += 64) {
+                        const double x = ca[k], y = cb[k];
+                        ca[k] = cc[u] * x - ss[u] * y;
+                        cb[k] = ss[u] * x + cc[u] * y;
+                    }
+                    if (qr) {
+                        const VP va = V + (long)pa[u] * m, vb = V + (long)pb[u] * m;
+                        for (int k = lane; k < m; k += 64) {
+                            const double x = va[k], y = vb[k];
+                            va[k] = cc[u] * x - ss[u] * y;
+                            vb[k] = ss[u] * x + cc[u] * y;
+                        }
+                    }
+                    rot = true;
+                }
             }
             __syncthreads();
         }
@@ -178,6 +214,117 @@ __device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, do
     return conv;
 }
 
+// Householder QR of T (w x m in LDS, ld w, w <= 512, w >= m) in place: R's part above the
+// diagonal in T, its diagonal in rdiag.  Every wavefront forms the reflector of a column by
+// itself (its rows in registers) and applies it to its share of the columns, so a column
+// takes one barrier.  The reflectors I - rtau v v^T stay as v(1:) = rsc times T's part below
+// the diagonal.  A barrier precedes the return.
+__device__ __forceinline__ void m2h_qr_lds(m2h_ldbl *T, int w, int m, double *rdiag, double *rsc, double *rtau)
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, NW = M2H_SVD_WG / 64;
+    for (int k = 0; k < m; k++) {
+        const m2h_ldbl *x = T + k + (long)k * w;
+        const int len = w - k;
+        double v[8], part = 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const int i = 1 + lane + 64 * q;
+            v[q] = i < len ? x[i] : 0.0;
+            part += v[q] * v[q];
+        }
+        const double xn = sqrt(team_bfly(part, 64)), alpha = x[0];
+        double diag = alpha, rs = 0.0, rt = 0.0;
+        if (xn != 0.0) {  // else H = I
+            const double beta = -copysign(hypot(alpha, xn), alpha);
+            const double tau = (beta - alpha) / beta, scal = 1.0 / (alpha - beta);
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] *= scal;
+            for (int j = k + 1 + wv; j < m; j += NW) {
+                m2h_ldbl *c = T + k + (long)j * w;
+                double cv[8], d = 0.0;
+                const double c0 = c[0];
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const int i = 1 + lane + 64 * q;
+                    cv[q] = i < len ? c[i] : 0.0;
+                    d += v[q] * cv[q];
+                }
+                d = (c0 + team_bfly(d, 64)) * tau;
+                if (lane == 0) c[0] = c0 - d;
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const int i = 1 + lane + 64 * q;
+                    if (i < len) c[i] = cv[q] - d * v[q];
+                }
+            }
+            diag = beta;
+            rs = scal;
+            rt = tau;
+        }
+        if (threadIdx.x == 0) { rdiag[k] = diag; rsc[k] = rs; rtau[k] = rt; }
+        __syncthreads();
+    }
+}
+
+// V := Q of the QR above for a square matrix (w = m <= 128): the reflectors applied to the
+// identity, a column per wavefront in registers, four columns at a time.
+__device__ __forceinline__ void m2h_q_form(const m2h_ldbl *T, m2h_ldbl *V, int m, const double *rsc, const double *rtau)
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, NW = M2H_SVD_WG / 64;
+    for (int j0 = wv; j0 < m; j0 += 4 * NW) {
+        double c[4][2];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) c[t][q] = lane + 64 * q == j0 + t * NW ? 1.0 : 0.0;
+        for (int k = m - 1; k >= 0; k--) {
+            const double sc = rsc[k], tau = rtau[k];
+            double v[2], d[4];
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int i = lane + 64 * q;
+                v[q] = i == k ? 1.0 : (i > k && i < m) ? T[i + k * m] * sc : 0.0;
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++) d[t] = team_bfly(v[0] * c[t][0] + v[1] * c[t][1], 64);
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int q = 0; q < 2; q++) c[t][q] -= d[t] * tau * v[q];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int i = lane + 64 * q, j = j0 + t * NW;
+                if (i < m && j < m) V[i + j * m] = c[t][q];
+            }
+    }
+}
+
+// One chunk of rows of a tall matrix (rows x m at src, ld lds) reduced to its R (m x m at
+// dst, ld ldd): the tree reduction that brings a context of thousands of rows down to what
+// k_m2h_svd holds in LDS.  One workgroup walking the whole matrix in global memory took
+// about 7 ms for 1936 x 64, with most CUs idle.
+struct M2hChunk { long src, dst; int rows, m, lds, ldd; };
+__global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_qr(const M2hChunk *ch, double *S)
+{
+    extern __shared__ double m2h_dyn[];
+    __shared__ double rdiag[M2H_QM], rsc[M2H_QM], rtau[M2H_QM];
+    const M2hChunk C = ch[blockIdx.x];
+    m2h_ldbl *T = (m2h_ldbl *)m2h_dyn;
+    const double *src = S + C.src;
+    double *dst = S + C.dst;
+    for (int e = threadIdx.x; e < C.rows * C.m; e += M2H_SVD_WG)
+        T[e] = src[(e % C.rows) + (long)(e / C.rows) * C.lds];
+    __syncthreads();
+    m2h_qr_lds(T, C.rows, C.m, rdiag, rsc, rtau);
+    for (int e = threadIdx.x; e < C.m * C.m; e += M2H_SVD_WG) {
+        const int i = e % C.m, j = e / C.m;
+        dst[i + (long)j * C.ldd] = i < j ? T[i + (long)j * C.rows] : i == j ? rdiag[j] : 0.0;
+    }
+}
+
 __global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_svd(const M2hJob *jobs, double *S, double *Bs, double tol, int *rank,
                                                         int *err, int lds_cap)
 {
@@ -195,7 +342,45 @@ __global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_svd(const M2hJob *jobs, doub
     const long rsz = (long)m * P;
     const bool rl = rsz <= lds_cap, vl = rl && qr && rsz + (long)m * m <= lds_cap;
     m2h_ldbl *Rl = (m2h_ldbl *)m2h_dyn, *Vl = Rl + rsz;
-    if (qr) {
+    if (qr && vl && w <= 512 && (long)w * m <= lds_cap) {
+        // The matrix itself in LDS, then R over it.  With lq the sweeps run on L = R3^T of a
+        // second QR, R^T = Q3 R3, with the rotations accumulated on Q3: T = Q L Q3^T, and the
+        // rows of R3 are graded, which takes 9 sweeps where R takes 21 (64 columns of the
+        // Cauchy test matrix).  Leaving pairs of columns below tol alone would save rotations,
+        // but near a spectrum that is dense around tol it never converges.
+        // Not for a sketch: its largest singular value is so much above the block's that
+        // eps sigma_1 is a sizeable part of tol, and another QR's rounding moves the rank.
+        __shared__ double rdiag[M2H_QM], rsc[M2H_QM], rtau[M2H_QM];
+        constexpr int NE = M2H_QM * M2H_QM / M2H_SVD_WG + 1;  // elements of an m x m matrix per thread
+        double r[NE];
+        for (int e = tid; e < w * m; e += M2H_SVD_WG) Rl[e] = T[e];
+        __syncthreads();
+        m2h_qr_lds(Rl, w, m, rdiag, rsc, rtau);
+        // the triangle a QR leaves (ld ldr) or its transpose to the front of the LDS
+        auto triangle = [&](int ldr, bool tr) {
+#pragma unroll
+            for (int q = 0; q < NE; q++) {
+                const int e = tid + q * M2H_SVD_WG, i = tr ? e / m : e % m, j = tr ? e % m : e / m;
+                r[q] = e < m * m ? (i < j ? Rl[i + j * ldr] : i == j ? rdiag[j] : 0.0) : 0.0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < NE; q++) {
+                const int e = tid + q * M2H_SVD_WG;
+                if (e < m * m) Rl[e] = r[q];
+            }
+            __syncthreads();
+        };
+        triangle(w, J.lq != 0);
+        if (J.lq) {
+            m2h_qr_lds(Rl, m, m, rdiag, rsc, rtau);
+            m2h_q_form(Rl, Vl, m, rsc, rtau);
+            __syncthreads();
+            triangle(m, true);
+        } else {
+            for (int e = tid; e < m * m; e += M2H_SVD_WG) Vl[e] = (e % m == e / m) ? 1.0 : 0.0;
+        }
+    } else if (qr) {
         for (int k = 0; k < m; k++) {
             double *x = T + k + (long)k * w;
             const int len = w - k;
@@ -244,9 +429,9 @@ __global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_svd(const M2hJob *jobs, doub
     __syncthreads();
     bool conv;
     m2h_gdbl *Rq = (m2h_gdbl *)Rg, *Vq = (m2h_gdbl *)Vg;
-    if (vl) conv = m2h_jacobi(Rl, Vl, qr, m, P, sv, ord, B, &s_rot);
-    else if (rl) conv = m2h_jacobi(Rl, Vq, qr, m, P, sv, ord, B, &s_rot);
-    else conv = m2h_jacobi(Rq, Vq, qr, m, P, sv, ord, B, &s_rot);
+    if (vl) conv = m2h_jacobi(Rl, Vl, qr, m, P, sv, ord, B, &s_rot, red);
+    else if (rl) conv = m2h_jacobi(Rl, Vq, qr, m, P, sv, ord, B, &s_rot, red);
+    else conv = m2h_jacobi(Rq, Vq, qr, m, P, sv, ord, B, &s_rot, red);
     if (!conv && tid == 0) atomicOr(err, 1);
     for (int j = tid; j < P; j += M2H_SVD_WG)
         if (sv[j] > tol) atomicAdd(&s_cnt, 1);
