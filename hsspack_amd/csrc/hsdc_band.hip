@@ -239,51 +239,69 @@ __global__ __launch_bounds__(BWG) void k_sb_split(const double *ab, int ldab, in
 // Cyclic two-sided Jacobi: each round's rotations come from the round's starting values
 // (|a_pq| > m eps sqrt|a_pp a_qq|), then all row rotations, all column rotations (and
 // the vectors), and the pairs' off-diagonal entries set to zero.  Eigenvalues ascending
-// into D (ties by index), vectors into Q's diagonal block, INDXQ = 1..m.
+// into D (ties by the selection sort), vectors into Q's diagonal block, INDXQ = 1..m.
+//
+// The bound is the latency of a round (m - 1 of them a sweep, about nine sweeps): sixteen
+// wavefronts take a pair each with a lane per element (four wavefronts before, finding
+// pair and element by integer division), the columns of A lie an odd distance apart so
+// that the row rotations do not conflict in LDS, and the vectors stay in LDS beside A up to
+// m = 98 (v_lds), else in Q.  A round of a 94-row leaf took 7 us before.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BWG) void k_sb_leaf(const double *ab, int ldab, int kd, int lower, const int *leaf_st,
-                                                 const int *leaf_m, int nleaf, const double *cuts, double *Q, long ldq,
-                                                 double *D, int *indxq, int *info)
+#define LEAF_WG 1024
+
+// (value, position) minimum over the wavefront, ties to the smaller position
+template <int O>
+__device__ __forceinline__ void leaf_min_step(double &v, int &p)
 {
-    extern __shared__ double A[];  // m x m
+    const double v2 = xlane<O>(v);
+    const int p2 = xlane32<O>(p);
+    if (v2 < v || (v2 == v && p2 < p)) { v = v2; p = p2; }
+}
+
+__global__ __launch_bounds__(LEAF_WG) void k_sb_leaf(const double *ab, int ldab, int kd, int lower, const int *leaf_st,
+                                                     const int *leaf_m, int nleaf, const double *cuts, double *Q,
+                                                     long ldq, double *D, int *indxq, int *info, int v_lds)
+{
+    extern __shared__ double A[];  // m x m, ld la; then the vectors likewise when v_lds
     __shared__ double rc[BLEAF_MAX / 2], rs[BLEAF_MAX / 2], dg[BLEAF_MAX];
     __shared__ int rp[BLEAF_MAX / 2], rq[BLEAF_MAX / 2], perm[BLEAF_MAX], np, rot;
-    const int i = blockIdx.x, st = leaf_st[i], m = leaf_m[i], tid = threadIdx.x;
+    const int i = blockIdx.x, st = leaf_st[i], m = leaf_m[i], tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    constexpr int NW = LEAF_WG / 64;
+    const int la = m | 1;
     const long cs = 2L * kd * kd + kd;
-    double *Qb = Q + st + (long)st * ldq;
-    for (int e = tid; e < m * m; e += BWG) {
-        const int r = e % m, c = e / m;
-        double a = band_at(ab, ldab, kd, lower, st + r, st + c);
-        if (i > 0 && r < kd && c < kd) {  // V S V^T of the cut before the leaf
-            const double *V = cuts + (long)(i - 1) * cs + kd * kd, *S = V + kd * kd;
-            double acc = 0.0;
-            for (int t = 0; t < kd; t++) acc += V[r + t * kd] * S[t] * V[c + t * kd];
-            a -= acc;
+    double *Qb = Q + st + (long)st * ldq, *Vl = A + la * m;
+    for (int c = wv; c < m; c += NW)
+        for (int r = lane; r < m; r += 64) {
+            double a = band_at(ab, ldab, kd, lower, st + r, st + c);
+            if (i > 0 && r < kd && c < kd) {  // V S V^T of the cut before the leaf
+                const double *V = cuts + (long)(i - 1) * cs + kd * kd, *S = V + kd * kd;
+                double acc = 0.0;
+                for (int t = 0; t < kd; t++) acc += V[r + t * kd] * S[t] * V[c + t * kd];
+                a -= acc;
+            }
+            if (i + 1 < nleaf && r >= m - kd && c >= m - kd) {  // U S U^T of the cut after it
+                const double *U = cuts + (long)i * cs, *S = U + 2 * kd * kd;
+                const int rr = r - (m - kd), cc = c - (m - kd);
+                double acc = 0.0;
+                for (int t = 0; t < kd; t++) acc += U[rr + t * kd] * S[t] * U[cc + t * kd];
+                a -= acc;
+            }
+            A[r + c * la] = a;
+            if (v_lds) Vl[r + c * la] = (r == c) ? 1.0 : 0.0;
+            else Qb[r + (long)c * ldq] = (r == c) ? 1.0 : 0.0;
         }
-        if (i + 1 < nleaf && r >= m - kd && c >= m - kd) {  // U S U^T of the cut after it
-            const double *U = cuts + (long)i * cs, *S = U + 2 * kd * kd;
-            const int rr = r - (m - kd), cc = c - (m - kd);
-            double acc = 0.0;
-            for (int t = 0; t < kd; t++) acc += U[rr + t * kd] * S[t] * U[cc + t * kd];
-            a -= acc;
-        }
-        A[e] = a;
-        Qb[r + (long)c * ldq] = (r == c) ? 1.0 : 0.0;
-    }
     __syncthreads();
     const int P = m + (m & 1);
     bool conv = false;
     for (int sweep = 0; sweep < 40 && !conv; sweep++) {
-        if (tid == 0) rot = 0;
+        if (tid == 0) { rot = 0; np = 0; }
         __syncthreads();
         for (int r = 0; r < P - 1; r++) {
-            if (tid == 0) np = 0;
-            __syncthreads();
             if (tid < P / 2) {
                 int p = rr_player(tid, r, P), q = rr_player(P - 1 - tid, r, P);
                 if (p > q) { int t = p; p = q; q = t; }
                 if (q < m) {
-                    const double apq = A[p + q * m], app = A[p + p * m], aqq = A[q + q * m];
+                    const double apq = A[p + q * la], app = A[p + p * la], aqq = A[q + q * la];
                     if (apq != 0.0 && fabs(apq) > m * HSDC_EPS * sqrt(fabs(app * aqq))) {
                         const double th = (aqq - app) / (2.0 * apq);
                         const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(1.0 + th * th));
@@ -295,57 +313,82 @@ __global__ __launch_bounds__(BWG) void k_sb_leaf(const double *ab, int ldab, int
             }
             __syncthreads();
             const int npp = np;
-            if (npp > 0) {
-                for (int e = tid; e < npp * m; e += BWG) {  // rows p, q
-                    const int k = e / m, j = e % m, p = rp[k], q = rq[k];
-                    const double c = rc[k], s = rs[k], x = A[p + j * m], y = A[q + j * m];
-                    A[p + j * m] = c * x - s * y;
-                    A[q + j * m] = s * x + c * y;
+            for (int k = wv; k < npp; k += NW) {  // rows p, q
+                const int p = rp[k], q = rq[k];
+                const double c = rc[k], s = rs[k];
+                for (int j = lane; j < m; j += 64) {
+                    const double x = A[p + j * la], y = A[q + j * la];
+                    A[p + j * la] = c * x - s * y;
+                    A[q + j * la] = s * x + c * y;
                 }
-                __syncthreads();
-                for (int e = tid; e < npp * m; e += BWG) {  // columns p, q of A and of the vectors
-                    const int k = e / m, ii = e % m, p = rp[k], q = rq[k];
-                    const double c = rc[k], s = rs[k];
-                    double x = A[ii + p * m], y = A[ii + q * m];
-                    A[ii + p * m] = c * x - s * y;
-                    A[ii + q * m] = s * x + c * y;
-                    double *qp = Qb + ii + (long)p * ldq, *qq = Qb + ii + (long)q * ldq;
-                    x = *qp;
-                    y = *qq;
-                    *qp = c * x - s * y;
-                    *qq = s * x + c * y;
-                }
-                __syncthreads();
-                for (int k = tid; k < npp; k += BWG) {
-                    A[rp[k] + rq[k] * m] = 0.0;
-                    A[rq[k] + rp[k] * m] = 0.0;
-                }
-                if (tid == 0) rot += npp;
             }
+            __syncthreads();
+            for (int k = wv; k < npp; k += NW) {  // columns p, q of A and of the vectors
+                const int p = rp[k], q = rq[k];
+                const double c = rc[k], s = rs[k];
+                for (int ii = lane; ii < m; ii += 64) {
+                    double x = A[ii + p * la], y = A[ii + q * la];
+                    // the pair's off-diagonal entries are zero
+                    A[ii + p * la] = ii == q ? 0.0 : c * x - s * y;
+                    A[ii + q * la] = ii == p ? 0.0 : s * x + c * y;
+                    if (v_lds) {
+                        x = Vl[ii + p * la];
+                        y = Vl[ii + q * la];
+                        Vl[ii + p * la] = c * x - s * y;
+                        Vl[ii + q * la] = s * x + c * y;
+                    } else {
+                        double *qp = Qb + ii + (long)p * ldq, *qq = Qb + ii + (long)q * ldq;
+                        x = *qp;
+                        y = *qq;
+                        *qp = c * x - s * y;
+                        *qq = s * x + c * y;
+                    }
+                }
+            }
+            if (tid == 0) { rot += npp; np = 0; }
             __syncthreads();
         }
         conv = (rot == 0);
         __syncthreads();
     }
     if (!conv && tid == 0) atomicOr(info, 1);
-    for (int j = tid; j < m; j += BWG) dg[j] = A[j + j * m];
+    for (int j = tid; j < m; j += LEAF_WG) dg[j] = A[j + j * la];
     __syncthreads();
-    if (tid == 0) {
-        for (int j = 0; j < m; j++) perm[j] = j;
+    if (wv == 0) {
+        // selection sort over positions a .. m - 1, the first smallest each time; lane l holds
+        // positions l and l + 64 (value and original column)
+        double v0 = lane < m ? dg[lane] : 0.0, v1 = lane + 64 < m ? dg[lane + 64] : 0.0;
+        int i0 = lane, i1 = lane + 64;
         for (int a = 0; a + 1 < m; a++) {
-            int k = a;
-            for (int j = a + 1; j < m; j++) if (dg[perm[j]] < dg[perm[k]]) k = j;
-            const int t = perm[a]; perm[a] = perm[k]; perm[k] = t;
+            const bool in0 = lane >= a && lane < m, in1 = lane + 64 >= a && lane + 64 < m;
+            double v = in0 ? v0 : in1 ? v1 : __builtin_huge_val();
+            int p = in0 ? lane : in1 ? lane + 64 : 1 << 20;
+            if (in0 && in1 && v1 < v0) { v = v1; p = lane + 64; }
+            leaf_min_step<32>(v, p);
+            leaf_min_step<16>(v, p);
+            leaf_min_step<8>(v, p);
+            leaf_min_step<4>(v, p);
+            leaf_min_step<2>(v, p);
+            leaf_min_step<1>(v, p);
+            const int k = p < m ? p : a;  // nothing below infinity: the position itself
+            const double va = __shfl(a < 64 ? v0 : v1, a & 63), vk = __shfl(k < 64 ? v0 : v1, k & 63);
+            const int ia = __shfl(a < 64 ? i0 : i1, a & 63), ik = __shfl(k < 64 ? i0 : i1, k & 63);
+            if (lane == (k & 63)) { if (k < 64) { v0 = va; i0 = ia; } else { v1 = va; i1 = ia; } }
+            if (lane == (a & 63)) { if (a < 64) { v0 = vk; i0 = ik; } else { v1 = vk; i1 = ik; } }
         }
+        if (lane < m) perm[lane] = i0;
+        if (lane + 64 < m) perm[lane + 64] = i1;
     }
     __syncthreads();
-    for (int e = tid; e < m * m; e += BWG) A[e] = Qb[(e % m) + (long)(e / m) * ldq];
-    __syncthreads();
-    for (int e = tid; e < m * m; e += BWG) {
-        const int r = e % m, c = e / m;
-        Qb[r + (long)c * ldq] = A[r + perm[c] * m];
+    if (!v_lds) {
+        for (int c = wv; c < m; c += NW)
+            for (int r = lane; r < m; r += 64) A[r + c * la] = Qb[r + (long)c * ldq];
+        __syncthreads();
     }
-    for (int j = tid; j < m; j += BWG) {
+    const double *V = v_lds ? Vl : A;
+    for (int c = wv; c < m; c += NW)
+        for (int r = lane; r < m; r += 64) Qb[r + (long)c * ldq] = V[r + perm[c] * la];
+    for (int j = tid; j < m; j += LEAF_WG) {
         D[st + j] = dg[perm[j]];
         indxq[st + j] = j + 1;
     }
@@ -1079,9 +1122,12 @@ int sb_solve(hsdc_sb_ctx *c, int lower, int n, int kd, const double *dab, long l
     for (int m : P.leaf_m) mmax = std::max(mmax, m);
     double *Qc[2] = {(double *)c->q[0].p, (double *)c->q[1].p};
     double *Zc[2] = {(double *)c->z[0].p, (double *)c->z[1].p};
-    hipLaunchKernelGGL(k_sb_leaf, dim3(nb), dim3(BWG), sizeof(double) * (size_t)mmax * mmax, st, dab, (int)ldab, kd,
-                       lower, (const int *)(tb + o_lst), (const int *)(tb + o_lm), nb, (const double *)cuts, Qc[0],
-                       (long)n, Dp[0], indxq, dinfo);
+    // A (columns an odd distance apart) and, where 160 KB of LDS hold them too, the vectors
+    const size_t la = sizeof(double) * (size_t)(mmax | 1) * mmax;
+    const int v_lds = 2 * la <= 156 * 1024;
+    hipLaunchKernelGGL(k_sb_leaf, dim3(nb), dim3(LEAF_WG), v_lds ? 2 * la : la, st, dab, (int)ldab, kd, lower,
+                       (const int *)(tb + o_lst), (const int *)(tb + o_lm), nb, (const double *)cuts, Qc[0], (long)n,
+                       Dp[0], indxq, dinfo, v_lds);
     SHK(hipGetLastError());
     // ---- merges
     hsdc_stats h0;  // the HSS context's totals before this solve (its figures are the change)
