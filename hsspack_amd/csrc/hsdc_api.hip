@@ -95,7 +95,6 @@ __global__ void k_m2h_copy(const M2hCopy *, const M2hJob *, const double *, cons
                            double *, double *);
 __global__ void k_cfill_general(int, const double *, const double *, const double *, const double *, double *);
 __global__ void k_hss_init(const HssMerge *);
-__global__ void k_hss_reset(const HssMerge *);
 __global__ void k_hss_dgen(const HssMerge *, const HssNode *, int);
 template <int NT, bool SQ>
 __global__ void k_hss_rowcomp(const HssMerge *, const HssNode *, int, double, int);
@@ -970,7 +969,6 @@ static int hss_apply(hsdc_ctx *c, const std::vector<HssSpec> &sp, int ni, double
             const size_t ldsb = sizeof(double) * (size_t)ldsn;
             const HssNode *sn = dN + step_off[st];
             const HssCompact *sc = dC + comp_off[st];
-            hipLaunchKernelGGL(k_hss_reset, dim3(nh), dim3(64), 0, s, dH);
             if (sq && nn < 512)
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hss_rowcomp<512, true>), dim3(nn), dim3(512), ldsb, s, dH, sn, nn,
                                    tol, ldsn);
@@ -984,7 +982,6 @@ static int hss_apply(hsdc_ctx *c, const std::vector<HssSpec> &sp, int ni, double
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hss_rowcomp<256, false>), dim3(nn), dim3(256), 0, s, dH, sn, nn, tol,
                                    0);
             hipLaunchKernelGGL(k_hss_compact, dim3(nc), dim3(WGS), 0, s, dH, sc, dO, 1);
-            hipLaunchKernelGGL(k_hss_reset, dim3(nh), dim3(64), 0, s, dH);
             if (sq && nn < 512)
                 hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hss_colcomp<512, true>), dim3(nn), dim3(512), ldsb, s, dH, sn, nn,
                                    tol, ldsn);

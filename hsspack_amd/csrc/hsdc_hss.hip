@@ -1335,6 +1335,7 @@ __global__ __launch_bounds__(WG) void k_hss_compact(const HssMerge *hm, const Hs
     const HssMerge H = hm[C.mrg];
     const int tid = threadIdx.x;
     int *rng = rows ? H.lr : H.lc;
+    if (tid == 0) *H.scratch_top = 0ULL;  // the next compression starts its private copies afresh
     if (*H.err) return;
     // the host builds trees of at most 512 leaves, so a compaction lists at most 1024
     // nodes; a larger one would not fit the slice table and sends the merge dense
@@ -1734,11 +1735,6 @@ __global__ __launch_bounds__(WG) void k_cbuild(const HssMerge *hm, int h, double
         if (H.sq) den = den * (A1(H.FF, i) + A1(H.D0, j));
         C[e] = A1(H.U0, i) * A1(H.V0, j) / den;
     }
-}
-
-__global__ void k_hss_reset(const HssMerge *hm)
-{
-    if (threadIdx.x == 0) *hm[blockIdx.x].scratch_top = 0ULL;
 }
 
 // 256 threads per node when a launch has nodes for every CU twice over, 512 when
