@@ -2412,7 +2412,7 @@ int hsdc_laed3(hsdc_ctx *c, int k, int n, int n1, double *d, double *q, int ldq,
     int info = 0;
     HK(hipMemcpy(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost));
     HK(hipMemcpy(d, W.lam, sizeof(double) * k, hipMemcpyDeviceToHost));
-    HK(hipMemcpy2D(q, sizeof(double) * ldq, Y, sizeof(double) * n, sizeof(double) * n, k, hipMemcpyDeviceToHost));
+    HK(copy_matrix(q, ldq, Y, n, n, k, hipMemcpyDeviceToHost));
     if (k >= 3) HK(hipMemcpy(w, W.wnew, sizeof(double) * k, hipMemcpyDeviceToHost));
     return info ? 1 : 0;
 }
@@ -2486,15 +2486,13 @@ static int hss_one(hsdc_ctx *c, int sq, int k, int ni, double tol, const double 
     if (left) {  // q is k x nrow: staged as is, transposed on the device into X^T (nrow x k)
         CK(ensure(c->tb, sizeof(double) * (size_t)std::max(nrow, 1) * k));
         if (nrow > 0) {
-            HK(hipMemcpy2D(c->tb.p, sizeof(double) * k, q, sizeof(double) * ldq, sizeof(double) * k, nrow,
-                           hipMemcpyHostToDevice));
+            HK(copy_matrix(c->tb.p, k, q, ldq, k, nrow, hipMemcpyHostToDevice));
             hipLaunchKernelGGL(k_transpose, dim3(cdiv(k, 64), cdiv(nrow, 64)), dim3(WGS), 0, s, k, nrow,
                                (const double *)c->tb.p, (long)k, (double *)c->xb.p, (long)nrow);
             HK(hipGetLastError());
         }
     } else {
-        HK(hipMemcpy2D(c->xb.p, sizeof(double) * nrow, q, sizeof(double) * ldq, sizeof(double) * nrow, k,
-                       hipMemcpyHostToDevice));
+        HK(copy_matrix(c->xb.p, nrow, q, ldq, nrow, k, hipMemcpyHostToDevice));
     }
     HssSpec sp;
     sp.K = k;
@@ -2510,12 +2508,10 @@ static int hss_one(hsdc_ctx *c, int sq, int k, int ni, double tol, const double 
             hipLaunchKernelGGL(k_transpose, dim3(cdiv(nrow, 64), cdiv(k, 64)), dim3(WGS), 0, s, nrow, k,
                                (const double *)c->yb.p, (long)nrow, (double *)c->tb.p, (long)k);
             HK(hipGetLastError());
-            HK(hipMemcpy2D(q, sizeof(double) * ldq, c->tb.p, sizeof(double) * k, sizeof(double) * k, nrow,
-                           hipMemcpyDeviceToHost));
+            HK(copy_matrix(q, ldq, c->tb.p, k, k, nrow, hipMemcpyDeviceToHost));
         }
     } else {
-        HK(hipMemcpy2D(q, sizeof(double) * ldq, c->yb.p, sizeof(double) * nrow, sizeof(double) * nrow, k,
-                       hipMemcpyDeviceToHost));
+        HK(copy_matrix(q, ldq, c->yb.p, nrow, nrow, k, hipMemcpyDeviceToHost));
     }
     if (ranks) {
         const HssPlanM &Q = keep[0];
@@ -2616,8 +2612,7 @@ int hsdc_cauchyhssmm(hsdc_ctx *c, const double *d, const double *f, const double
     for (int i = 0; i < 4; i++) HK(hipMemcpyAsync(gd + i * nn, hsrc[i], sizeof(double) * nn, hipMemcpyHostToDevice, s));
     CK(ensure(c->q, sizeof(double) * nn * nn));
     double *dB = (double *)c->q.p;
-    HK(hipMemcpy2DAsync(dB, sizeof(double) * nn, b, sizeof(double) * ldb, sizeof(double) * nn, nn,
-                        hipMemcpyHostToDevice, s));
+    HK(copy_matrix_async(dB, nn, b, ldb, nn, nn, hipMemcpyHostToDevice, s));
     std::vector<HssPlanM> P(1);
     HssPlanM &Q = P[0];
     Q.ok = false;
@@ -2743,8 +2738,7 @@ int hsdc_cauchyhssmm(hsdc_ctx *c, const double *d, const double *f, const double
         HK(hipGetLastError());
     }
     HK(hipEventRecord(c->ev1, s));
-    HK(hipMemcpy2DAsync(b, sizeof(double) * ldb, dB, sizeof(double) * nn, sizeof(double) * nn, nn,
-                        hipMemcpyDeviceToHost, s));
+    HK(copy_matrix_async(b, ldb, dB, nn, nn, nn, hipMemcpyDeviceToHost, s));
     HK(hipStreamSynchronize(s));
     float ms_mm = 0.0f;
     (void)hipEventElapsedTime(&ms_mm, c->ev0, c->ev1);
@@ -3054,14 +3048,12 @@ static int dhss_run(hsdc_ctx *c, const double *a, int lda, int n, double *b, int
     const size_t nn = (size_t)n, kk = (size_t)k;
     CK(ensure(c->zout, sizeof(double) * nn * nn));
     double *dA = (double *)c->zout.p;
-    HK(hipMemcpy2DAsync(dA, sizeof(double) * nn, a, sizeof(double) * lda, sizeof(double) * nn, nn,
-                        hipMemcpyHostToDevice, s));
+    HK(copy_matrix_async(dA, nn, a, lda, nn, nn, hipMemcpyHostToDevice, s));
     // b on the device: n x k (left) or k x n, leading dimension its row count
     const size_t br = left ? nn : kk, bc = left ? kk : nn;
     CK(ensure(c->q, sizeof(double) * br * bc));
     double *dB = (double *)c->q.p;
-    HK(hipMemcpy2DAsync(dB, sizeof(double) * br, b, sizeof(double) * ldb, sizeof(double) * br, bc,
-                        hipMemcpyHostToDevice, s));
+    HK(copy_matrix_async(dB, br, b, ldb, br, bc, hipMemcpyHostToDevice, s));
     std::vector<HssPlanM> P(1);
     float ms_build = 0.0f;
     CK(mat2hss_build(c, dA, n, ni, tol, P[0], ranks, &ms_build, rsvd, seed));
@@ -3106,8 +3098,7 @@ static int dhss_run(hsdc_ctx *c, const double *a, int lda, int n, double *b, int
         HK(hipGetLastError());
     }
     HK(hipEventRecord(c->ev1, s));
-    HK(hipMemcpy2DAsync(b, sizeof(double) * ldb, dB, sizeof(double) * br, sizeof(double) * br, bc,
-                        hipMemcpyDeviceToHost, s));
+    HK(copy_matrix_async(b, ldb, dB, br, br, bc, hipMemcpyDeviceToHost, s));
     HK(hipStreamSynchronize(s));
     float ms_mm = 0.0f;
     (void)hipEventElapsedTime(&ms_mm, c->ev0, c->ev1);
@@ -3185,18 +3176,15 @@ int hsdc_laed0(hsdc_ctx *c, int icompq, int qsiz, int n, double *d, double *e, d
     if (info) return info;
     HK(hipMemcpy(d, dd, sizeof(double) * n, hipMemcpyDeviceToHost));
     if (icompq == 2) {
-        HK(hipMemcpy2D(q, sizeof(double) * ldq, dz, sizeof(double) * n, sizeof(double) * n, n,
-                       hipMemcpyDeviceToHost));
+        HK(copy_matrix(q, ldq, dz, n, n, n, hipMemcpyDeviceToHost));
     } else if (icompq == 1) {
         CK(ensure(c->misc, sizeof(double) * 2 * (size_t)qsiz * n));
         double *qa = (double *)c->misc.p, *qc = qa + (size_t)qsiz * n;
-        HK(hipMemcpy2D(qa, sizeof(double) * qsiz, q, sizeof(double) * ldq, sizeof(double) * qsiz, n,
-                       hipMemcpyHostToDevice));
+        HK(copy_matrix(qa, qsiz, q, ldq, qsiz, n, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(k_dgemm_nn, dim3(cdiv(qsiz, 64), cdiv(n, 64)), dim3(WGS), 0, c->stream, qsiz, n, n,
                            (const double *)qa, (long)qsiz, (const double *)dz, (long)n, qc, (long)qsiz);
         HK(hipGetLastError());
-        HK(hipMemcpy2D(q, sizeof(double) * ldq, qc, sizeof(double) * qsiz, sizeof(double) * qsiz, n,
-                       hipMemcpyDeviceToHost));
+        HK(copy_matrix(q, ldq, qc, qsiz, qsiz, n, hipMemcpyDeviceToHost));
     }
     return 0;
 }
@@ -3249,8 +3237,7 @@ int hsdc_stedc(hsdc_ctx *c, char compz, int n, double *d, double *e, double *z, 
         // COMPZ = 'V': Z := Zin * Q (the back-transformation of DSTEDC) on the device
         CK(ensure(c->misc, sizeof(double) * 2 * (size_t)n * n));
         double *za = (double *)c->misc.p, *zc = za + (size_t)n * n;
-        HK(hipMemcpy2D(za, sizeof(double) * n, z, sizeof(double) * ldz, sizeof(double) * n, n,
-                       hipMemcpyHostToDevice));
+        HK(copy_matrix(za, n, z, ldz, n, n, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(k_dgemm_nn, dim3(cdiv(n, 64), cdiv(n, 64)), dim3(WGS), 0, c->stream, n, n, n,
                            (const double *)za, (long)n, (const double *)dz, (long)n, zc, (long)n);
         HK(hipGetLastError());

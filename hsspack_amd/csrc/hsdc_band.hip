@@ -1476,8 +1476,7 @@ int hsdc_sbevd(hsdc_sb_ctx *c, char compz, char uplo, int n, int kd, const doubl
     if (info < 0) return info;
     SHK(hipMemcpyAsync(d, dd, sizeof(double) * n, hipMemcpyDeviceToHost, st));
     if (vec)
-        SHK(hipMemcpy2DAsync(q, sizeof(double) * ldq, dq, sizeof(double) * n, sizeof(double) * n, n,
-                             hipMemcpyDeviceToHost, st));
+        SHK(copy_matrix_async(q, ldq, dq, n, n, n, hipMemcpyDeviceToHost, st));
     SHK(hipStreamSynchronize(st));
     return info;
 }

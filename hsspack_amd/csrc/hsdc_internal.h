@@ -155,3 +155,19 @@ struct SecCtl {
     int kmin;                    // merges with k < kmin use (and harvest) the classical start only
     float gate;                  // the proposal is taken when |log-correction| > gate
 };
+
+// A rows x cols column-major matrix of doubles between host and device (columns ldd and lds
+// apart), queued on s, or waited for on the null stream.  Contiguous on both sides it goes
+// as one linear copy: HIP copies a 2-D block of pageable memory column by column, 32 MB in
+// 17 ms where the linear copy takes 1 ms up and 2 ms down.
+inline hipError_t copy_matrix_async(void *dst, long ldd, const void *src, long lds, long rows, long cols,
+                                    hipMemcpyKind kind, hipStream_t s)
+{
+    if (ldd == rows && lds == rows) return hipMemcpyAsync(dst, src, sizeof(double) * (size_t)rows * cols, kind, s);
+    return hipMemcpy2DAsync(dst, sizeof(double) * ldd, src, sizeof(double) * lds, sizeof(double) * rows, cols, kind, s);
+}
+inline hipError_t copy_matrix(void *dst, long ldd, const void *src, long lds, long rows, long cols, hipMemcpyKind kind)
+{
+    if (ldd == rows && lds == rows) return hipMemcpy(dst, src, sizeof(double) * (size_t)rows * cols, kind);
+    return hipMemcpy2D(dst, sizeof(double) * ldd, src, sizeof(double) * lds, sizeof(double) * rows, cols, kind);
+}

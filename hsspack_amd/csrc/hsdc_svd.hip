@@ -2315,10 +2315,8 @@ int hsdc_bdsdc(hsdc_bd_ctx *c, char uplo, char compq, int n, double *d, double *
     if (info) return info;
     BHK(hipMemcpyAsync(d, dd, sizeof(double) * n, hipMemcpyDeviceToHost, st));
     if (icompq == 2) {
-        BHK(hipMemcpy2DAsync(u, sizeof(double) * ldu, du, sizeof(double) * n, sizeof(double) * n, n,
-                             hipMemcpyDeviceToHost, st));
-        BHK(hipMemcpy2DAsync(vt, sizeof(double) * ldvt, dvt, sizeof(double) * n, sizeof(double) * n, n,
-                             hipMemcpyDeviceToHost, st));
+        BHK(copy_matrix_async(u, ldu, du, n, n, n, hipMemcpyDeviceToHost, st));
+        BHK(copy_matrix_async(vt, ldvt, dvt, n, n, n, hipMemcpyDeviceToHost, st));
     }
     BHK(hipStreamSynchronize(st));
     return 0;
