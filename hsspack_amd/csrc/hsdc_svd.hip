@@ -1093,17 +1093,32 @@ __device__ __forceinline__ double bd_acol(const BdWork &W, const BdMerge &M, con
 }
 
 // ------------------------------------------------------------------------------
-// DLASD3's products U(:,1:K) = U2 Bu, V(:,1:K) = VT2^T Bv: 64 x 64 output tiles, 16
-// inner indices staged per step, each output summed over the inner index in
-// ascending order
+// DLASD3's products U(:,1:K) = U2 Bu, V(:,1:K) = VT2^T Bv: 64 x 64 output tiles, each
+// output summed over the inner index in ascending order (multiply and add rounded
+// apart, so no matrix instruction).  A tile lists the columns whose support meets its
+// rows, BG_K of the merge at a time and in order; about half of them are the other
+// child's, zero in every row here, and a zero product leaves a sum that began at +0 as
+// it is.  The list holds what a staged element would look up again (slot, support).
+// 16 entries a chunk go through two LDS slabs, the next one's loads in flight while
+// this one multiplies; a chunk's elements of B are read along its columns.  A level of
+// the 16384 SVDs: 513 -> 240 us where little deflates (bound by the multiplies and adds,
+// K to 1024), 55 -> 31 us where K is about 60 (bound by the latency of the few chunks).
 // ------------------------------------------------------------------------------
+#define BG_K 512
+#define BG_P 65
+static __device__ double bdg_zero = 0.0;  // what a staged element outside the operands reads
+typedef const __attribute__((address_space(1))) double bgdbl;
 __global__ __launch_bounds__(256) void k_bd_gemm(const BdMerge *mg, int nmg, BdTab tab, BdWork W, const BdOut *mo,
                                                  const double *Q, const double *U, const double *V, long ld,
                                                  double *stg)
 {
-  __shared__ double As[16][65];
-  __shared__ double Bs[16][65];
+  __shared__ double As[2][16 * BG_P], Bs[2][16 * BG_P];
+  __shared__ long l_col[BG_K];                      // offset of the column's row 0 (global) in X
+  __shared__ int l_lo[BG_K], l_hi[BG_K], l_j[BG_K];  // its row support, its index
+  __shared__ int wcnt[2][4];
   const int ttot = tab.tile[nmg];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  bgdbl *const zero = (bgdbl *)&bdg_zero;
   for (int bi = blockIdx.x; bi < ttot; bi += gridDim.x) {
     // tiles of a merge: for every 64 output columns, the U row tiles then the V row tiles
     const int mi = bd_find(tab.tile, nmg, bi);
@@ -1116,37 +1131,110 @@ __global__ __launch_bounds__(256) void k_bd_gemm(const BdMerge *mg, int nmg, BdT
     const int row0 = (isV ? rem - ntu : rem) * 64, col0 = (lt / (ntu + ntv)) * 64;
     const int rows = isV ? m : n;
     const double *X = isV ? V : U;
+    const int *slot = (isV ? W.gV : W.gU) + M.s, *slo = (isV ? W.gVlo : W.gUlo) + M.s,
+              *shi = (isV ? W.gVhi : W.gUhi) + M.s;
     double *Y = stg + tab.soff[2 * mi + (isV ? 1 : 0)];
     const double *B = Q + tab.qoff[mi] + (isV ? (long)k * k : 0);
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int tx = tid & 15, ty = tid >> 4;
+    const int row = row0 + lane, grow = M.s + row;  // this thread's staged row of A
+    const bool rok = row < rows;
     double acc[4][4];
+#pragma unroll
     for (int a = 0; a < 4; a++)
+#pragma unroll
         for (int c = 0; c < 4; c++) acc[a][c] = 0.0;
-    for (int j0 = 0; j0 < k; j0 += 16) {
-        for (int e = threadIdx.x; e < 1024; e += 256) {
-            int rr = e & 63, jj = e >> 6;
-            int r = row0 + rr, J = j0 + jj;
-            As[jj][rr] = (r < rows && J < k) ? bd_acol(W, M, o, isV, X, ld, J, r) : 0.0;
-            int cc = e & 63, j2 = e >> 6;
-            int col = col0 + cc, J2 = j0 + j2;
-            Bs[j2][cc] = (col < k && J2 < k) ? B[(long)col * k + J2] : 0.0;
+    for (int g0 = 0; g0 < k; g0 += BG_K) {
+        int gn = 0;
+        __syncthreads();  // the list and the slabs of the previous tile or group are free
+#pragma unroll
+        for (int h = 0; h < BG_K / 256; h++) {
+            const int J = g0 + 256 * h + tid;
+            int sl = 0, lo = 0, hi = 0;
+            if (J < k) {
+                if (J == 0) {  // the special first column: row nl of U; of V rows 0..nl, or all
+                    lo = isV ? M.s : M.s + M.nl;
+                    hi = isV && m > n ? M.s + m : M.s + M.nl + 1;
+                } else {
+                    sl = slot[J]; lo = slo[J]; hi = shi[J];
+                }
+            }
+            const bool in = lo < hi && lo < M.s + row0 + 64 && hi > M.s + row0;
+            const unsigned long long bal = __ballot(in);
+            if (lane == 0) wcnt[h][wv] = __popcll(bal);
+            __syncthreads();
+            int at = gn;
+            for (int w = 0; w < 4; w++) {
+                if (w < wv) at += wcnt[h][w];
+                gn += wcnt[h][w];
+            }
+            if (in) {
+                at += __popcll(bal & ((1ULL << lane) - 1));
+                l_col[at] = (long)sl * ld; l_lo[at] = lo; l_hi[at] = hi; l_j[at] = J;
+            }
         }
         __syncthreads();
-        const int jn = min(16, k - j0);
-        for (int jj = 0; jj < jn; jj++) {
-            double av[4], bv[4];
-            for (int a = 0; a < 4; a++) av[a] = As[jj][tx + 16 * a];
-            for (int c = 0; c < 4; c++) bv[c] = Bs[jj][ty + 16 * c];
-            for (int a = 0; a < 4; a++)
-                for (int c = 0; c < 4; c++) acc[a][c] = acc[a][c] + av[a] * bv[c];
-        }
+        if (gn == 0) continue;
+        double ra[4], rb[4];
+        auto stage = [&](int k0) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int t = k0 + wv + 4 * e, tc = min(t, gn - 1);
+                bgdbl *pa = (bgdbl *)X + (l_col[tc] + grow);
+                ra[e] = *(t < gn && rok && grow >= l_lo[tc] && grow < l_hi[tc] ? pa : zero);
+            }
+            const int t = k0 + tx, tc = min(t, gn - 1), J = l_j[tc];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int col = col0 + ty + 16 * e;
+                bgdbl *pb = (bgdbl *)B + ((long)col * k + J);
+                rb[e] = *(t < gn && col < k ? pb : zero);
+            }
+            if (g0 + k0 + wv == 0 && l_j[0] == 0) ra[0] = rok ? bd_acol(W, M, o, isV, X, ld, 0, row) : 0.0;
+        };
+        auto commit = [&](int h) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                As[h][(wv + 4 * e) * BG_P + lane] = ra[e];
+                Bs[h][tx * BG_P + ty + 16 * e] = rb[e];
+            }
+        };
+        stage(0);
+        commit(0);
         __syncthreads();
+        int h = 0;
+        for (int k0 = 0; k0 < gn; k0 += 16) {
+            const bool more = k0 + 16 < gn;
+            if (more) stage(k0 + 16);
+            const int ksteps = min(16, ((gn - k0) + 3) & ~3);
+            for (int kq = 0; kq < ksteps; kq += 4) {
+#pragma unroll
+                for (int jj = 0; jj < 4; jj++) {
+                    const double *ap = As[h] + (kq + jj) * BG_P + tx, *bp = Bs[h] + (kq + jj) * BG_P + ty;
+                    double av[4], bv[4];
+#pragma unroll
+                    for (int a = 0; a < 4; a++) av[a] = ap[16 * a];
+#pragma unroll
+                    for (int c = 0; c < 4; c++) bv[c] = bp[16 * c];
+#pragma unroll
+                    for (int a = 0; a < 4; a++)
+#pragma unroll
+                        for (int c = 0; c < 4; c++) acc[a][c] = acc[a][c] + av[a] * bv[c];
+                }
+            }
+            if (more) {
+                h ^= 1;
+                commit(h);
+            }
+            __syncthreads();
+        }
     }
+#pragma unroll
     for (int a = 0; a < 4; a++) {
-        int r = row0 + tx + 16 * a;
+        const int r = row0 + tx + 16 * a;
         if (r >= rows) continue;
+#pragma unroll
         for (int c = 0; c < 4; c++) {
-            int col = col0 + ty + 16 * c;
+            const int col = col0 + ty + 16 * c;
             if (col < k) Y[(long)col * rows + r] = acc[a][c];
         }
     }

@@ -94,3 +94,23 @@ def test_svd_fold_edges_bitexact(torch_dev, n):
     assert info == 0
     r = O.bdsdc(d, e)
     assert np.array_equal(s, r["d"]) and np.array_equal(u, r["u"]) and np.array_equal(vt, r["vt"])
+
+
+@pytest.mark.parametrize("n,uplo", [(511, "U"), (513, "L"), (1023, "L"), (1025, "U"), (1091, "L")])
+def test_svd_vector_products(torch_dev, n, uplo):
+    """The products of the singular vectors gather the columns of a merge 512 at a time
+    and only those that meet a tile's rows: almost no deflation, so the top merge's K lies
+    on both sides of 512 and 1024; the same bits as the oracle's full sums."""
+    rng = np.random.default_rng(n)
+    d, e = 2.0 + 0.01 * rng.uniform(size=n), 1.0 + 0.01 * rng.uniform(size=n - 1)
+    from hsspack_amd import hsdc
+    c = hsdc.BdContext()
+    try:
+        s, u, vt, info = c.bdsdc(d, e, uplo=uplo)
+        assert info == 0 and c.trace()["k"].max() > 0.9 * n
+    finally:
+        c.close()
+    r = O.bdsdc(d, e, uplo=uplo.encode())
+    np.testing.assert_array_equal(s, r["d"])
+    np.testing.assert_array_equal(u, r["u"])
+    np.testing.assert_array_equal(vt, r["vt"])
