@@ -55,7 +55,6 @@ __global__ void k_newcols_copy(const Merge *, const int *, int, int, const int *
 __global__ void k_lvltab(const Merge *, int, const MergeOut *, Work, LvlTab, long, long, int *);
 __global__ void k_final(const Prob *, const int *, Work, const int *, double *, const long *, const long *, int,
                         double *, const double *, unsigned long long *, const int *, int, int, int);
-__global__ void k_zfill(double *, long, long, long);
 __global__ void k_dgemm_nn(int, int, int, const double *, long, const double *, long, double *, long);
 __global__ void k_transpose(int, int, const double *, long, double *, long);
 #define C2H_WG 512     // threads of k_cauchy2hss
@@ -1565,7 +1564,7 @@ static int solve(hsdc_ctx *c, Plan &pl, const double *hd, const double *he, doub
             HK(hipEventRecord(c->zev0, s));
             HK(hipStreamWaitEvent(c->zstream, c->zev0, 0));
             if (c->prm.profile) HK(hipEventRecord(c->pz0, c->zstream));
-            hipLaunchKernelGGL(k_zfill, dim3(32768), dim3(WGS), 0, c->zstream, dZ, (long)ntot, (long)ntot, ldz[0]);
+            hipLaunchKernelGGL(k_zfill, dim3(ZF_BLOCKS), dim3(WGS), 0, c->zstream, dZ, (long)ntot, (long)ntot, ldz[0]);
             HK(hipGetLastError());
             if (c->prm.profile) HK(hipEventRecord(c->pz1, c->zstream));
             HK(hipEventRecord(c->zev1, c->zstream));

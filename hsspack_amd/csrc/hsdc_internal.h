@@ -171,3 +171,11 @@ inline hipError_t copy_matrix(void *dst, long ldd, const void *src, long lds, lo
     if (ldd == rows && lds == rows) return hipMemcpy(dst, src, sizeof(double) * (size_t)rows * cols, kind);
     return hipMemcpy2D(dst, sizeof(double) * ldd, src, sizeof(double) * lds, sizeof(double) * rows, cols, kind);
 }
+
+// Blocks of the zero fill beside a solve, 10 on each XCD: few enough not to hold up the
+// levels, enough to end before them up to n of about 45000.  DSTEDC of uniform spectra at
+// n = 16384, 32768, 40960 and 65536, ms: 2.35, 3.36, 4.01, 9.45 with 64 blocks, 2.34, 3.40,
+// 4.00, 8.12 with 80, 2.33, 3.49, 4.07, 7.71 with 96, 2.37, 3.93, 4.57, 7.63 with 128, and
+// 2.44, 4.40, 5.54, 10.1 with 32768 of 16-byte stores.
+#define ZF_BLOCKS 80
+__global__ void k_zfill(double *Z, long rows, long ncols, long ldz);

@@ -1994,21 +1994,22 @@ __global__ __launch_bounds__(LT_NT) void k_lvltab(const Merge *mg, int nm, const
 
 // ---------------------------------------------------------------------------
 // Zero fill of the rows x ncols output Z (leading dimension ldz), launched on a
-// second stream when the solve starts: the DC levels are latency bound and leave
-// HBM idle, so the 8 n^2 bytes of zeros are written under them, and the final
-// reordering writes only the supported rows.  Consecutive blocks write
-// consecutive 4 KB pieces (one contiguous front, as a plain device fill).
+// second stream when the solve starts: the levels are latency bound and leave HBM
+// idle, so the 8 n^2 bytes of zeros are written under them, and the final reordering
+// writes only the supported rows.  What the fill takes from the levels counts, not its
+// own time: from 32768 blocks with 16-byte stores it took 1.5 ms for n = 32768, but 7
+// kernels that need 40 us by themselves took 1.1 ms beside it.  So few blocks (ZF_BLOCKS)
+// and 8-byte stores, together a rate of about 4 TB/s that leaves the other memory traffic
+// through; 16-byte stores from as few blocks are worse than the full fill (4.67 ms for
+// the solve against 4.40, and 3.40 with 8-byte ones), write-through stores between the
+// two (3.9).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(WG) void k_zfill(double *Z, long rows, long ncols, long ldz)
 {
-    typedef double dbl2 __attribute__((ext_vector_type(2)));
-    const dbl2 z2 = {0.0, 0.0};
-    if (ldz == rows && (((unsigned long)Z) & 15) == 0) {
-        const long n2 = rows * ncols;
-        dbl2 *d2 = (dbl2 *)Z;
-        for (long q = blockIdx.x * (long)WG + threadIdx.x; q < (n2 >> 1); q += (long)gridDim.x * WG)
-            __builtin_nontemporal_store(z2, d2 + q);
-        if ((n2 & 1) && blockIdx.x == 0 && threadIdx.x == 0) Z[n2 - 1] = 0.0;
+    if (ldz == rows) {
+        const long tot = rows * ncols;
+        for (long q = blockIdx.x * (long)WG + threadIdx.x; q < tot; q += (long)gridDim.x * WG)
+            __builtin_nontemporal_store(0.0, Z + q);
     } else {
         for (long col = blockIdx.x; col < ncols; col += gridDim.x)
             for (long r = threadIdx.x; r < rows; r += WG) __builtin_nontemporal_store(0.0, Z + col * ldz + r);

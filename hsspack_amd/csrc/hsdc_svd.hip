@@ -1507,15 +1507,6 @@ __global__ __launch_bounds__(POST_NT) void k_bd_post(const BdMerge *mg, BdWork W
 // output: zeros everywhere (second stream, beside the levels), then column i of U
 // and row i of VT from the slot of virtual column perm(i), supported rows only
 // ------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_bd_zero(double *A, long lda, int n)
-{
-    const long tot = (long)n * n;
-    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < tot; e += (long)gridDim.x * 256) {
-        const long c = e / n, r = e - c * n;
-        A[c * lda + r] = 0.0;
-    }
-}
-
 __global__ __launch_bounds__(256) void k_bd_fin(const BdWork W, const double *Us, const double *Vs, long ld,
                                                 const int *perm, int n, double *U, long ldu)
 {
@@ -1920,8 +1911,8 @@ static int bd_solve(hsdc_bd_ctx *c, int n, const std::vector<double> &he, double
     if (dU || dVT) {
         BHK(hipEventRecord(c->ev[2], st));
         BHK(hipStreamWaitEvent(c->zstream, c->ev[2], 0));
-        if (dU) hipLaunchKernelGGL(k_bd_zero, dim3(8192), dim3(256), 0, c->zstream, dU, ldu, n);
-        if (dVT) hipLaunchKernelGGL(k_bd_zero, dim3(8192), dim3(256), 0, c->zstream, dVT, ldvt, n);
+        if (dU) hipLaunchKernelGGL(k_zfill, dim3(ZF_BLOCKS), dim3(256), 0, c->zstream, dU, (long)n, (long)n, ldu);
+        if (dVT) hipLaunchKernelGGL(k_zfill, dim3(ZF_BLOCKS), dim3(256), 0, c->zstream, dVT, (long)n, (long)n, ldvt);
         BHK(hipGetLastError());
         BHK(hipEventRecord(c->ev[3], c->zstream));
     }
@@ -2146,8 +2137,8 @@ static int bd_solve(hsdc_bd_ctx *c, int n, const std::vector<double> &he, double
     auto write_vectors = [&](bool clear) -> int {
         if (!(dU || dVT)) return 0;
         if (clear) {
-            if (dU) hipLaunchKernelGGL(k_bd_zero, dim3(8192), dim3(256), 0, st, dU, ldu, n);
-            if (dVT) hipLaunchKernelGGL(k_bd_zero, dim3(8192), dim3(256), 0, st, dVT, ldvt, n);
+            if (dU) hipLaunchKernelGGL(k_zfill, dim3(32768), dim3(256), 0, st, dU, (long)n, (long)n, ldu);
+            if (dVT) hipLaunchKernelGGL(k_zfill, dim3(32768), dim3(256), 0, st, dVT, (long)n, (long)n, ldvt);
         } else {
             BHK(hipStreamWaitEvent(st, c->ev[3], 0));
         }
