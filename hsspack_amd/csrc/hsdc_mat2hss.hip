@@ -6,9 +6,11 @@
 //
 //   k_m2h_gather   its block row (its rows against the other active columns) transposed
 //                  and its block column, as tall matrices (context x own)
+//   k_m2h_qr       contexts of many rows reduced first by a tree of QRs in LDS
 //   k_m2h_svd      one workgroup per (node, side): Householder QR of the tall matrix and
-//                  one-sided Jacobi on R's columns with the rotations accumulated (the
-//                  right singular vectors); for a matrix wider than tall the columns of
+//                  one-sided Jacobi, on the transposed triangle of a second QR or, for a
+//                  sketch, on R's columns with the rotations accumulated (the right
+//                  singular vectors); for a matrix wider than tall the columns of
 //                  its transpose are orthogonalised directly; the singular values
 //                  descending, the rank = their count above tol (mat2hssvd's
 //                  count(svs > tol)), the basis vectors in that order
