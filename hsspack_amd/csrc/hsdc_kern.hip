@@ -1999,9 +1999,9 @@ __global__ __launch_bounds__(LT_NT) void k_lvltab(const Merge *mg, int nm, const
 // writes only the supported rows.  What the fill takes from the levels counts, not its
 // own time: from 32768 blocks with 16-byte stores it took 1.5 ms for n = 32768, but 7
 // kernels that need 40 us by themselves took 1.1 ms beside it.  So few blocks (ZF_BLOCKS)
-// and 8-byte stores, 1.9 ms at 4.6 TB/s, that leave the other memory traffic through; 16-byte stores from as few blocks are worse than the full fill (4.67 ms for
-// the solve against 4.40, and 3.40 with 8-byte ones), write-through stores between the
-// two (3.9).
+// and 8-byte stores, 1.9 ms at 4.6 TB/s, that leave the other memory traffic through;
+// 16-byte stores from as few blocks are worse than the full fill (4.67 ms for the solve
+// against 4.40, and 3.40 with 8-byte ones), write-through stores between the two (3.9).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(WG) void k_zfill(double *Z, long rows, long ncols, long ldz)
 {
