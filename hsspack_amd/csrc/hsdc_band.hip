@@ -911,7 +911,7 @@ void sb_plan(SbPlan &P, int n, int kd, int smlsiz)
         P.leaf_st[i] = i ? lend[i - 1] : 0;
         P.leaf_m[i] = lend[i] - P.leaf_st[i];
     }
-    P.cut_ic.assign(nb > 1 ? nb - 1 : 0, 0);
+    P.cut_ic.assign(std::max(nb - 1, 1), 0);  // one leaf: an unused entry, the uploaded table is never empty
     for (int i = 0; i + 1 < nb; i++) P.cut_ic[i] = lend[i];
     P.lv.clear();
     int subpbs = nb;
@@ -1042,7 +1042,7 @@ int sb_solve(hsdc_sb_ctx *c, int lower, int n, int kd, const double *dab, long l
     };
     const size_t o_lst = put(P.leaf_st.data(), sizeof(int) * nb);
     const size_t o_lm = put(P.leaf_m.data(), sizeof(int) * nb);
-    const size_t o_cut = put(P.cut_ic.data(), sizeof(int) * std::max(nb - 1, 1));
+    const size_t o_cut = put(P.cut_ic.data(), sizeof(int) * P.cut_ic.size());
     struct LvOff { size_t mg, mg2, rc, cc, xo, so; int nrowb, ncol; };
     std::vector<LvOff> lo(nlv);
     for (int l = 0; l < nlv; l++) {

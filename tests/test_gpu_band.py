@@ -109,6 +109,19 @@ def test_dense_vs_oracle(torch_dev, n, kd):
     assert orth <= 1e-12 and res <= 1e-12
 
 
+@pytest.mark.parametrize("n,kd", [(1, 1), (2, 1), (40, 3), (98, 9), (99, 20), (128, 64)])
+def test_one_leaf(torch_dev, n, kd):
+    """An order within the leaf bound: no cut, no merge, one Jacobi leaf."""
+    ab = band_cfg(n, kd, seed=6, sub=n)
+    A = band_dense(ab)
+    rc, lam, q, st, tr = dev_solve(torch_dev, ab, kd)
+    assert rc == 0 and len(tr["k"]) == 0
+    w = np.linalg.eigvalsh(A)
+    assert np.abs(lam - w).max() <= 4 * n * EPS * np.abs(w).max()
+    assert np.abs(q.T @ q - np.eye(n)).max() <= 1e-12
+    assert np.abs(A @ q - q * lam).max() <= 1e-12 * np.abs(A).max()
+
+
 def test_lower_storage_and_host_entry(torch_dev):
     from hsspack_amd import hsdc
     n, kd = 333, 7
