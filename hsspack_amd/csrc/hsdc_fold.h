@@ -14,6 +14,7 @@
 // wavefront); K = 1400 dense vectors 182 -> 18 us.  Chunks of 32 poles (three blocks per
 // CU instead of two): 1.45 ms at K = 32768.
 #pragma once
+#include <algorithm>
 #include "hsdc_internal.h"
 
 #define OF_P 64    // poles per chunk
@@ -26,23 +27,29 @@ struct FoldLds {
 };
 
 // How a level's nch chunks of 256 roots are split over blocks: `parts` blocks to a chunk,
-// each taking the chunk's roots R at a time from its own part.  64 roots keep all eight
-// wavefronts' lanes on divides and is the faster split once the level fills the chip with
-// such blocks (two per CU, 128 chunks); below that, 16 roots per block give four times
-// the blocks, and a chunk costs the folding wavefront's steps instead of the divides.
+// each taking the chunk's roots R at a time from its own part.  Blocks of 16 roots are
+// four times as many, and a chunk of poles costs them the folding wavefront's steps instead
+// of the divides: the faster split as long as every one of them has a CU to itself, 16
+// chunks on 256 CUs.  From 17 on two would share a CU, and 64 roots, which keep all eight
+// wavefronts' lanes on divides, are faster.  One merge of K roots (secular equation, product
+// and norms), 16 against 64 roots, us: K = 2040 151 / 175, 4000 338 / 389, 4090 344 / 399,
+// 4500 529 / 486, 6000 717 / 657, 12000 2040 / 1658, 16384 3660 / 2710, 25000 8516 / 6250,
+// 32500 13124 / 9300.
 // From 1024 chunks on (many small merges) a block takes whole chunks: finding a part's
 // merge costs two dependent loads, more than the work of a part that is empty (2048
 // chunks of K = 40: 112 us against 422 for the vector build; 800 chunks of K = 500: 420
 // against 480 the other way round).
+#define OF_NARROW 16  // chunks up to which a block takes 16 roots
 struct FoldSplit { int R, parts; };
 __device__ __forceinline__ FoldSplit fold_split(int nch)
 {
-    return nch >= 1024 ? FoldSplit{64, 1} : nch >= 128 ? FoldSplit{64, 4} : FoldSplit{16, 16};
+    return nch >= 1024 ? FoldSplit{64, 1} : nch > OF_NARROW ? FoldSplit{64, 4} : FoldSplit{16, 16};
 }
-// Blocks to launch for at most nch chunks of 256 roots (the kernels stride)
+// Blocks to launch for at most nch chunks of 256 roots (the kernels stride): enough for the
+// narrow split too, which fewer chunks than the bound may take
 inline int fold_grid(long nch)
 {
-    const long b = nch >= 1024 ? nch : nch >= 128 ? 4 * nch : 16 * nch;
+    const long b = nch >= 1024 ? nch : nch > OF_NARROW ? std::max(4 * nch, 16L * OF_NARROW) : 16 * nch;
     return (int)(b < 1 ? 1 : b > 2048 ? 2048 : b);
 }
 
@@ -56,7 +63,7 @@ inline int fold_grid(long nch)
 //   fold(acc, t)     the fold
 // Every thread of the block calls it; n is uniform.  A block barrier precedes the
 // return, so the LDS may be reused at once.
-// r0: the block's first root (0-based).
+// r0: the block's first root (0-based).  n >= 1.
 template <int R, int NV, class F>
 __device__ __forceinline__ double ordered_fold(const F &f, int n, int r0, double acc, FoldLds<NV> &S)
 {

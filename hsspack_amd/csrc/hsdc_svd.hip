@@ -1004,7 +1004,7 @@ __device__ __forceinline__ void bd_loewner_block(int k, int s, int r0, const BdW
     BdLoewnerTerm f{W.dsg + s, W.tau + s, W.org + s, 0.0, i};
     f.di = f.ds[ic - 1];
     double zi = sv_den(f.di, f.ds[f.org[k - 1] - 1], f.tau[k - 1]);
-    zi = ordered_fold<R>(f, k - 1, r0, zi, S);
+    zi = ordered_fold<R>(f, k - 1, r0, zi, S);  // k >= 2: the level table lists no other merge
     if (threadIdx.x >= 512 && lane < R && i <= k) {
         const double a = sqrt(fabs(zi));
         W.zl[s + i - 1] = W.zs[s + i - 1] >= 0.0 ? a : -a;

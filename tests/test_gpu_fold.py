@@ -1,6 +1,6 @@
 """The ordered folds (Loewner products, column norms) at the edges of their splits: chunks
 of 64 poles, 16 or 64 roots per block, and the three ways a level's 256-root chunks are
-divided over blocks (below 128, from 128 and from 1024 chunks).  The fold keeps the pole
+divided over blocks (up to 16, from 17 and from 1024 chunks).  The fold keeps the pole
 order, so every value equals the oracle's bit for bit, and a batch's problems equal the
 same problems solved alone."""
 import numpy as np
@@ -28,7 +28,7 @@ def ctx(torch_dev):
     c.close()
 
 
-@pytest.mark.parametrize("K", [3, 15, 16, 17, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 1025])
+@pytest.mark.parametrize("K", [3, 15, 16, 17, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 1025, 4096, 4097])
 def test_loewner_and_alpha_edges_bitexact(ctx, K):
     rng = np.random.default_rng(K)
     d = np.sort(rng.uniform(-1, 1, K))
@@ -44,7 +44,7 @@ def test_loewner_and_alpha_edges_bitexact(ctx, K):
 
 @pytest.mark.parametrize("K", [33000])
 def test_wide_split_of_one_merge(torch_dev, ctx, K):
-    """At least 128 chunks (64 roots per block): the roots' Loewner identity, z unchanged up
+    """More than 128 chunks (64 roots per block): the roots' Loewner identity, z unchanged up
     to rounding (a product of K correctly rounded quotients: relative error <= 2 K eps) and
     unit columns."""
     rng = np.random.default_rng(1)
