@@ -249,7 +249,8 @@ __global__ __launch_bounds__(BWG) void k_sb_split(const double *ab, int ldab, in
 // ---------------------------------------------------------------------------
 #define LEAF_WG 1024
 
-// (value, position) minimum over the wavefront, ties to the smaller position
+// a step of the (value, position) minimum over the wavefront, ties to the smaller position
+// (no NaN among the values)
 template <int O>
 __device__ __forceinline__ void leaf_min_step(double &v, int &p)
 {
@@ -356,21 +357,27 @@ __global__ __launch_bounds__(LEAF_WG) void k_sb_leaf(const double *ab, int ldab,
     __syncthreads();
     if (wv == 0) {
         // selection sort over positions a .. m - 1, the first smallest each time; lane l holds
-        // positions l and l + 64 (value and original column)
+        // positions l and l + 64 (value and original column).  A NaN is below nothing and
+        // nothing is below it: it stays where it is at position a and is passed over
+        // elsewhere.  So the candidates hold numbers only, every lane ends with the same
+        // position, and the columns stay a permutation.
         double v0 = lane < m ? dg[lane] : 0.0, v1 = lane + 64 < m ? dg[lane + 64] : 0.0;
         int i0 = lane, i1 = lane + 64;
+        const double inf = __builtin_huge_val();
         for (int a = 0; a + 1 < m; a++) {
-            const bool in0 = lane >= a && lane < m, in1 = lane + 64 >= a && lane + 64 < m;
-            double v = in0 ? v0 : in1 ? v1 : __builtin_huge_val();
-            int p = in0 ? lane : in1 ? lane + 64 : 1 << 20;
-            if (in0 && in1 && v1 < v0) { v = v1; p = lane + 64; }
+            const bool c0 = lane >= a && lane < m && (v0 == v0 || lane == a);
+            const bool c1 = lane + 64 >= a && lane + 64 < m && (v1 == v1 || lane + 64 == a);
+            const double w0 = v0 == v0 ? v0 : -inf, w1 = v1 == v1 ? v1 : -inf;
+            double v = c0 ? w0 : c1 ? w1 : inf;
+            int p = c0 ? lane : c1 ? lane + 64 : 1 << 20;
+            if (c0 && c1 && w1 < w0) { v = w1; p = lane + 64; }
             leaf_min_step<32>(v, p);
             leaf_min_step<16>(v, p);
             leaf_min_step<8>(v, p);
             leaf_min_step<4>(v, p);
             leaf_min_step<2>(v, p);
             leaf_min_step<1>(v, p);
-            const int k = p < m ? p : a;  // nothing below infinity: the position itself
+            const int k = __builtin_amdgcn_readfirstlane(p);  // position a is always a candidate
             const double va = __shfl(a < 64 ? v0 : v1, a & 63), vk = __shfl(k < 64 ? v0 : v1, k & 63);
             const int ia = __shfl(a < 64 ? i0 : i1, a & 63), ik = __shfl(k < 64 ? i0 : i1, k & 63);
             if (lane == (k & 63)) { if (k < 64) { v0 = va; i0 = ia; } else { v1 = va; i1 = ia; } }
