@@ -24,6 +24,7 @@
 // The generators land in the layout the HSS multiply reads (U, V^T, B, D per node, the
 // post-ordered tree of npart), so DHSSMM and DHSSMML run the same batched multiply as
 // the eigenvector matrices.
+#include <float.h>
 #include <math.h>
 #include "hsdc_internal.h"
 
@@ -98,7 +99,8 @@ typedef __attribute__((address_space(1))) double m2h_gdbl;
 
 // Jacobi on the P columns of R (length m, ld m), with V when qr; then the singular values
 // (column norms) to sv, their descending order (ties by index) to ord, the basis to B.
-// Returns false when the sweeps did not converge.
+// Returns false when the sweeps did not converge or the matrix's norm is no finite number
+// (B, sv and ord may then be unset).
 template <class RP, class VP>
 __device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, double *sv, int *ord, double *B,
                                            int *s_rot, double *s_part)
@@ -117,6 +119,10 @@ __device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, do
     __syncthreads();
     double lim = 0.0;
     for (int q = 0; q < NW; q++) lim += s_part[q];
+    // A NaN, an infinity or an overflow among the squares: no angles and no order of the
+    // singular values; the caller multiplies densely.  Rotations keep the sum, so a norm
+    // below is a number whenever this test passes.
+    if (!(lim <= DBL_MAX)) return false;
     lim *= 0x1p-600;
     for (int sweep = 0; sweep < 60 && !conv; sweep++) {
         if (tid == 0) *s_rot = 0;
@@ -193,10 +199,16 @@ __device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, do
         if (lane == 0) sv[j] = q;
     }
     __syncthreads();
+    // positions by counting, ties by index: a permutation because the keys are totally ordered
+    // (a NaN would be the smallest)
+    auto key = [&](int j) { const double q = sv[j]; return q >= 0.0 ? q : -1.0; };
     for (int j = tid; j < P; j += M2H_SVD_WG) {
-        const double x = sv[j];
+        const double x = key(j);
         int rk = 0;
-        for (int i = 0; i < P; i++) rk += (sv[i] > x || (sv[i] == x && i < j)) ? 1 : 0;
+        for (int i = 0; i < P; i++) {
+            const double y = key(i);
+            rk += (y > x || (y == x && i < j)) ? 1 : 0;
+        }
         ord[rk] = j;
     }
     __syncthreads();
@@ -434,7 +446,10 @@ __global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_svd(const M2hJob *jobs, doub
     if (vl) conv = m2h_jacobi(Rl, Vl, qr, m, P, sv, ord, B, &s_rot, red);
     else if (rl) conv = m2h_jacobi(Rl, Vq, qr, m, P, sv, ord, B, &s_rot, red);
     else conv = m2h_jacobi(Rq, Vq, qr, m, P, sv, ord, B, &s_rot, red);
-    if (!conv && tid == 0) atomicOr(err, 1);
+    if (!conv) {  // uniform; the host then reads neither the rank nor the basis
+        if (tid == 0) { atomicOr(err, 1); rank[blockIdx.x] = 0; }
+        return;
+    }
     for (int j = tid; j < P; j += M2H_SVD_WG)
         if (sv[j] > tol) atomicAdd(&s_cnt, 1);
     __syncthreads();

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import oracle_py as O
+from test_oracle_dhssmm import fmm_matrix
 
 pytestmark = pytest.mark.gpu
 
@@ -20,6 +21,14 @@ def torch_dev():
 def sb(torch_dev):
     from hsspack_amd import hsdc
     c = hsdc.SbContext()
+    yield c
+    c.close()
+
+
+@pytest.fixture(scope="module")
+def ctx(torch_dev):
+    from hsspack_amd import hsdc
+    c = hsdc.Context()
     yield c
     c.close()
 
@@ -60,3 +69,34 @@ def test_band_leaf_nan_beside_rotations(sb, n, kd):
         assert info == 0 and np.isnan(w).sum() == 1, p
         assert np.abs(np.sort(w[~np.isnan(w)]) - want).max() <= 4 * n * 2.0 ** -53 * np.abs(want).max()
         assert np.linalg.matrix_rank(q) == n
+
+
+def same_product(y, ref, rel):
+    """The same entries are NaN or infinite, the others agree."""
+    fin = np.isfinite(ref)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
+    np.testing.assert_array_equal(y[np.isinf(ref)], ref[np.isinf(ref)])
+    assert fin.any() and np.abs(y[fin] - ref[fin]).max() <= rel * np.abs(ref[fin]).max()
+
+
+@pytest.mark.parametrize("n,ni", [(300, 40), (330, 99), (420, 130), (500, 160), (151, 100), (900, 60)])
+@pytest.mark.parametrize("seed", [None, 7])
+def test_dense_to_hss_product(ctx, n, ni, seed):
+    """A NaN, an infinity or squares that overflow in an off-diagonal block leave no singular
+    values to order, with R and V in LDS, R alone or neither, for contexts wider and narrower
+    than the block and after a tree of QRs: the product is taken densely.  On a leaf's diagonal
+    block the form is built as ever, and the leaf's rows carry the value."""
+    a0 = fmm_matrix(n, 5)
+    b = np.random.default_rng(n).uniform(0.5, 1, (n, 30))
+    for at, x in (((n - 1, 0), np.nan), ((0, n - 1), np.inf), ((n // 4, 3 * n // 4), -np.inf), ((1, 0), np.nan)):
+        a = a0.copy()
+        a[at] = x
+        y, _, ranks = ctx.dhssmm(a, b, ni, 1e-11, seed=seed)
+        assert (ranks is None) == (at != (1, 0)), at
+        same_product(y, a @ b, 1e-9)
+    y, _, ranks = ctx.dhssmm(a0 * 2.0 ** 520, b, ni, 1e-11, seed=seed)
+    assert ranks is None
+    same_product(y, (a0 @ b) * 2.0 ** 520, 1e-12)
+    y, _, ranks = ctx.dhssmm(a0, b, ni, 1e-11, seed=seed)
+    assert ranks is not None
+    same_product(y, a0 @ b, 1e-9)
