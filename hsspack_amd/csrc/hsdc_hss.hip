@@ -212,9 +212,12 @@ __device__ __forceinline__ int scan_lanes(int k, int NTH)
     while (g < 64 && 2 * g * k <= NTH) g *= 2;
     return g;
 }
-// (value, smallest index) maximum over aligned groups of g lanes
+// (value, smallest index) maximum over aligned groups of g lanes, the same in every lane of
+// a group: values >= 0, a NaN counts as the smallest (compared as it is, it would stay in
+// its own lane, and the lanes would go on with different columns)
 __device__ __forceinline__ VI group_argmax(VI x, int g)
 {
+    if (!(x.v >= 0.0)) x.v = -1.0;
     if (g > 32) x = vi_step<32>(x);
     if (g > 16) x = vi_step<16>(x);
     if (g > 8) x = vi_step<8>(x);

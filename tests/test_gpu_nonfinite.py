@@ -100,3 +100,29 @@ def test_dense_to_hss_product(ctx, n, ni, seed):
     y, _, ranks = ctx.dhssmm(a0, b, ni, 1e-11, seed=seed)
     assert ranks is not None
     same_product(y, a0 @ b, 1e-9)
+
+
+@pytest.mark.parametrize("K,ni", [(513, 64), (1500, 64), (1500, 256)])
+def test_structured_product_with_a_nan(ctx, K, ni):
+    """A NaN among the row generators stays one row of the Schur complements: the swap check's
+    lanes must agree on every column's largest entry all the same.  Every entry of the product
+    sums over that row; the call after it is as if the NaN had not been."""
+    rng = np.random.default_rng(K)
+    d = np.sort(rng.uniform(-1, 1, K))
+    z = rng.standard_normal(K)
+    z /= np.linalg.norm(z)
+    v = O.mdlaed3_vectors(d, z, 1.1)
+    x = rng.uniform(0.5, 1, (9, K))
+
+    def product(zz):
+        return ctx.hss_evc(v["dlamda"], v["d"], zz, v["alpha"], v["difl"], v["difr"], x, ni, 1e-14)
+
+    want, ranks = product(v["z"])
+    for p in (0, 70, K // 2, K - 1):
+        zz = v["z"].copy()
+        zz[p] = np.nan
+        y, _ = product(zz)
+        assert np.isnan(y).all(), p
+    again, ranks2 = product(v["z"])
+    np.testing.assert_array_equal(again, want)
+    np.testing.assert_array_equal(ranks2, ranks)
