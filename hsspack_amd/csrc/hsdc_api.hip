@@ -18,6 +18,7 @@
 #include "hsdc_internal.h"
 #include "hsdc_hss.h"
 #include "hsdc_hss_host.h"
+#include "hsdc_m2h.h"
 
 #define HSS_LDS_V 16384  // doubles of dynamic LDS for an RRLU node's generator column
 #include "hsdc_mlp.h"
@@ -57,41 +58,6 @@ __global__ void k_final(const Prob *, const int *, Work, const int *, double *, 
                         double *, const double *, unsigned long long *, const int *, int, int, int);
 __global__ void k_dgemm_nn(int, int, int, const double *, long, const double *, long, double *, long);
 __global__ void k_transpose(int, int, const double *, long, double *, long);
-#define C2H_WG 512     // threads of k_cauchy2hss
-#define C2H_LDS 18432  // LDS doubles it may take
-__global__ void k_cauchy2hss(C2H, int);
-struct M2hJob {
-    int rs, rn, cs, cn;
-    int w, m;
-    long toff;
-    long boff;
-    int lq;
-};
-struct M2hBlk {
-    int start, count;
-    int src;
-    int ostart, ocount;
-};
-struct M2hCopy {
-    int kind, rows, cols, job;
-    int r0, c0;
-    long dst;
-};
-__global__ void k_m2h_gather(const M2hJob *, const double *, long, double *);
-#define M2H_SVD_WG 1024     // threads per block of k_m2h_svd
-#define M2H_LDS 19800       // LDS doubles it may take (160 KB less its static arrays)
-__global__ void k_m2h_svd(const M2hJob *, double *, double *, double, int *, int *, int);
-struct M2hChunk { long src, dst; int rows, m, lds, ldd; };
-__global__ void k_m2h_qr(const M2hChunk *, double *);
-// rows of an m-column matrix that one workgroup reduces in LDS (0: more columns than the
-// tree reduction takes; at least 2 m, so every stage shrinks the matrix)
-static int m2h_qr_rows(int m) { return m < 1 || m > 96 ? 0 : std::min(512, M2H_LDS / m); }
-__global__ void k_m2h_sketch(const M2hJob *, const M2hJob *, const double *, double *, unsigned long long);
-__global__ void k_m2h_rows(const M2hBlk *, int, const M2hJob *, const double *, const double *, long, int, double *,
-                           long);
-__global__ void k_m2h_cols(const M2hBlk *, int, const M2hJob *, const double *, const double *, long, int, double *);
-__global__ void k_m2h_copy(const M2hCopy *, const M2hJob *, const double *, const double *, long, const double *, long,
-                           double *, double *);
 __global__ void k_cfill_general(int, const double *, const double *, const double *, const double *, double *);
 __global__ void k_hss_init(const HssMerge *);
 __global__ void k_hss_dgen(const HssMerge *, const HssNode *, int);

@@ -55,6 +55,10 @@ struct C2H {
     unsigned long long *nswap;   // swaps of the RRLU
 };
 
+#define C2H_WG 512     // threads of k_cauchy2hss
+#define C2H_LDS 18432  // LDS doubles it may take
+__global__ void k_cauchy2hss(C2H C, int lds_cap);
+
 // One node of one merge's post-ordered HSS tree (aux_hss.f90:737-800).
 struct HssNode {
     int mrg;        // index into the HssMerge table

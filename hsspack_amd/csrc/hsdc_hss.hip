@@ -1769,9 +1769,7 @@ template __global__ void k_hss_colcomp<512, true>(const HssMerge *, const HssNod
 // pass, and W, needed only by the swap check and the generator, is formed ten steps at a
 // time with a thread per entry.  n = 2000, leaf 64: 50.7 ms before, 17.2 now.
 // ===========================================================================
-#define C2H_WG 512
 #define C2H_NW (C2H_WG / 64)
-#define C2H_LDS 18432  // doubles of dynamic LDS
 
 // first largest |U(i) / (X(i) - y)| over i = k .. n (index i - k + 1), i from i0 by step
 template <class DP>

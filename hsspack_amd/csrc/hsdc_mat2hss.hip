@@ -27,6 +27,7 @@
 #include <float.h>
 #include <math.h>
 #include "hsdc_internal.h"
+#include "hsdc_m2h.h"
 
 #define MWG 256
 
@@ -39,17 +40,6 @@ __device__ __forceinline__ int m2h_rr(int slot, int r, int P)
 }
 
 }  // namespace
-
-// One node's compression problem of one side: T (w x m, column-major, ld w) gathered
-// from C; the result basis (m x m, ld m, columns in descending singular value order),
-// its singular values and rank.  side 0: block row (basis U), 1: block column (W).
-struct M2hJob {
-    int rs, rn, cs, cn;  // the node's rows and columns in C
-    int w, m;            // context length and own length of this side
-    long toff;           // T, then R (m x m), V (m x m) at toff + w m, + m m
-    long boff;           // basis (m x m) and singular values (m)
-    int lq;              // 1: a second QR before the Jacobi sweeps
-};
 
 // ---------------------------------------------------------------------------
 // Gather the tall matrices: side 0: T(o, t) = C(rs + t, col_o), col_o the o-th column
@@ -91,9 +81,6 @@ __global__ __launch_bounds__(MWG) void k_m2h_gather(const M2hJob *jobs, const do
 // wavefronts and R and V in global memory a level of the n = 2000, leaf 64 matrix took
 // 26 ms.
 // ---------------------------------------------------------------------------
-#define M2H_SVD_WG 1024
-#define M2H_QM 100  // columns of a QR in LDS (R and V both fit up to 99)
-
 typedef __attribute__((address_space(3))) double m2h_ldbl;
 typedef __attribute__((address_space(1))) double m2h_gdbl;
 
@@ -228,10 +215,10 @@ __device__ __forceinline__ bool m2h_jacobi(RP R, VP V, bool qr, int m, int P, do
     return conv;
 }
 
-// Householder QR of T (w x m in LDS, ld w, w <= 512, w >= m) in place: R's part above the
-// diagonal in T, its diagonal in rdiag.  Every wavefront forms the reflector of a column by
-// itself (its rows in registers) and applies it to its share of the columns, so a column
-// takes one barrier.  The reflectors I - rtau v v^T stay as v(1:) = rsc times T's part below
+// Householder QR of T (w x m in LDS, ld w, m <= w <= M2H_QR_ROWS, m <= M2H_QM) in place: R's
+// part above the diagonal in T, its diagonal in rdiag.  Every wavefront forms the reflector
+// of a column by itself (its rows in registers) and applies it to its share of the columns,
+// so a column takes one barrier.  The reflectors I - rtau v v^T stay as v(1:) = rsc times T's part below
 // the diagonal.  A barrier precedes the return.
 __device__ __forceinline__ void m2h_qr_lds(m2h_ldbl *T, int w, int m, double *rdiag, double *rsc, double *rtau)
 {
@@ -320,7 +307,6 @@ __device__ __forceinline__ void m2h_q_form(const m2h_ldbl *T, m2h_ldbl *V, int m
 // dst, ld ldd): the tree reduction that brings a context of thousands of rows down to what
 // k_m2h_svd holds in LDS.  One workgroup walking the whole matrix in global memory took
 // about 7 ms for 1936 x 64, with most CUs idle.
-struct M2hChunk { long src, dst; int rows, m, lds, ldd; };
 __global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_qr(const M2hChunk *ch, double *S)
 {
     extern __shared__ double m2h_dyn[];
@@ -356,7 +342,7 @@ __global__ __launch_bounds__(M2H_SVD_WG) void k_m2h_svd(const M2hJob *jobs, doub
     const long rsz = (long)m * P;
     const bool rl = rsz <= lds_cap, vl = rl && qr && rsz + (long)m * m <= lds_cap;
     m2h_ldbl *Rl = (m2h_ldbl *)m2h_dyn, *Vl = Rl + rsz;
-    if (qr && vl && w <= 512 && (long)w * m <= lds_cap) {
+    if (qr && vl && w <= M2H_QR_ROWS && (long)w * m <= lds_cap) {
         // The matrix itself in LDS, then R over it.  With lq the sweeps run on L = R3^T of a
         // second QR, R^T = Q3 R3, with the rotations accumulated on Q3: T = Q L Q3^T, and the
         // rows of R3 are graded, which takes 9 sweeps where R takes 21 (64 columns of the
@@ -499,12 +485,6 @@ __global__ __launch_bounds__(MWG) void k_m2h_sketch(const M2hJob *jobs, const M2
 
 // New rows of C: for each new row block a, U_q^T C(rows of q, :) when it comes from a
 // job pair q (src >= 0), the old rows otherwise.  out is nnr x nc (ld nnr).
-struct M2hBlk {
-    int start, count;  // new block in C' (rows or columns)
-    int src;           // >= 0: job pair (2 src = row side, 2 src + 1 = column side); < 0: -1 - old block
-    int ostart, ocount;  // the old rows / columns it is formed from
-};
-
 __global__ __launch_bounds__(MWG) void k_m2h_rows(const M2hBlk *blk, int nb, const M2hJob *jobs, const double *Bs,
                                                   const double *C, long ldc, int nc, double *out, long ldo)
 {
@@ -558,14 +538,7 @@ __global__ __launch_bounds__(MWG) void k_m2h_cols(const M2hBlk *blk, int nb, con
     }
 }
 
-// Copies of one level's generators into the arena: kind 0 U (m x r from the row basis),
-// 1 V = W^T (r x m from the column basis), 2 B (a block of C'), 3 D (a block of A).
-struct M2hCopy {
-    int kind, rows, cols, job;  // job: the basis (kinds 0, 1)
-    int r0, c0;                 // the block's origin in its source (kinds 2, 3)
-    long dst;                   // arena / leaf-block offset
-};
-
+// Copies of one level's generators into the arena (M2hCopy).
 __global__ __launch_bounds__(MWG) void k_m2h_copy(const M2hCopy *cp, const M2hJob *jobs, const double *Bs,
                                                   const double *Cn, long ldcn, const double *A, long lda,
                                                   double *arena, double *dd)
