@@ -465,7 +465,7 @@ __global__ __launch_bounds__(MWG) void k_m2h_sketch(const M2hJob *jobs, const M2
                                                     unsigned long long seed)
 {
     const M2hJob J = jobs[blockIdx.y], K = sk[blockIdx.y];
-    if (K.w == J.w) return;  // no sketch for this side
+    if (K.lq) return;  // no sketch for this side (a tree of QRs may have changed its width)
     const int side = blockIdx.y & 1, pp = K.w, w = J.w;
     const double *T = S0 + J.toff;
     double *Y = S + K.toff;
