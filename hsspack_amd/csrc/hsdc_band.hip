@@ -245,7 +245,7 @@ __global__ __launch_bounds__(BWG) void k_sb_split(const double *ab, int ldab, in
 // wavefronts take a pair each with a lane per element (four wavefronts before, finding
 // pair and element by integer division), the columns of A lie an odd distance apart so
 // that the row rotations do not conflict in LDS, and the vectors stay in LDS beside A up to
-// m = 98 (v_lds), else in Q.  A round of a 94-row leaf took 7 us before.
+// m = 99 (v_lds), else in Q.  A round of a 94-row leaf took 7 us before.
 // ---------------------------------------------------------------------------
 #define LEAF_WG 1024
 

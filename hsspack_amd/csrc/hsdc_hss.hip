@@ -310,7 +310,8 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_rowcomp(const HssMerge *hm, con
 {
     extern __shared__ double hss_dyn[];  // lds_cap doubles: V when the node's columns fit
     __shared__ double F[HSS_MAXM], A[HSS_MAXM], Z[HSS_MAXM], W[HSS_MAXM];
-    __shared__ double T1[HSS_MAXM], T2[HSS_MAXM];  // factors of thread 0's ordered products
+    // factors of the ordered products: W(k) on the last wavefront, the swap on thread 0
+    __shared__ double T1[HSS_MAXM], T2[HSS_MAXM];
     __shared__ int PL[HSS_MAXM], PUs[HSS_MAXM];
     __shared__ short PQ[HSS_MAXM], IP[HSS_MAXM];   // positions within the node (<= HSS_MAXM)
     __shared__ VI red[4 * (HSS_CWG / 64)];
@@ -801,7 +802,7 @@ __global__ __launch_bounds__(HSS_CWG) void k_hss_colcomp(const HssMerge *hm, con
 {
     extern __shared__ double hss_dyn[];  // lds_cap doubles: V when the node's rows fit
     __shared__ double Dr[HSS_MAXM], A[HSS_MAXM], Z[HSS_MAXM], W[HSS_MAXM];
-    // factors of thread 0's ordered products; during the swap check's scan, the scanned
+    // factors of the ordered products, as in the row compression; in the swap check the scanned
     // rows' root data
     __shared__ double T12[2 * HSS_MAXM];
     double *const T1 = T12, *const T2 = T12 + HSS_MAXM;
