@@ -37,7 +37,7 @@ HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFS = 78.6
 # HBM bytes per k_zfill launch measured with rocprofv3 FETCH_SIZE / WRITE_SIZE passes, calibrated on a
 # 1 GiB device copy (profiles/k_zfill_n32768_uniform_traffic.md); keyed by (generator, n, seed)
-K_ZFILL_TRAFFIC = {(2, 32768, 2): (97 + 8396163) * 1024}
+K_ZFILL_TRAFFIC = {(2, 32768, 2): (40 + 8388627) * 1024}
 GEN = {1: "d=2+U(-1e-3,1e-3), e=1+U(-1e-3,1e-3)", 2: "d,e~U(-1,1)"}
 
 
@@ -249,7 +249,7 @@ def bench_tridiag(args, np, torch, hsdc, cfg, n, seed, tol, d, e, steps, warmup,
                                     "unit_note": "16 B per (i, j) operand pair, K^2 per merge for the products, "
                                                  "K^2 more per HSS merge for alpha; the operands are staged in LDS, "
                                                  "so this is an operand rate in HBM units, not HBM traffic: the "
-                                                 "sweeps are bound by the FP64 divides of one thread per root"}
+                                                 "sweeps are bound by the FP64 divides"}
     if sp["hss_mm_flops"] and acc["ms_hss_mm"] > 0:
         tf = sp["hss_mm_flops"] / (acc["ms_hss_mm"] * 1e-3) / 1e12
         hot["k_bgemm"] = {"flops": sp["hss_mm_flops"], "ms": acc["ms_hss_mm"], "TFLOPs": tf,
