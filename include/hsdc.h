@@ -224,7 +224,8 @@ int hsdc_cauchyhssmm(hsdc_ctx *ctx, const double *d, const double *f, const doub
  * time or more.  a is not modified (the reference uses it as workspace); prank is
  * accepted and unused, as in mat2hssvd.  time[0..1] (may be NULL): construction and
  * multiplication seconds; ranks (may be NULL; 2 per tree node): the ranks of each node's
- * U and V, or ranks[0] = -1 when A was applied densely.  INFO: -i for an illegal
+ * U and V, or ranks[0] = -1 when A was applied densely (a tree of one leaf, or a block
+ * with a NaN, an infinity or squares that overflow).  INFO: -i for an illegal
  * argument i (-1 a, -2 lda, -3 m != n, -4 n, -5 b, -6 ldb, -7 k, -8 tol, -10 ni, -11 ncol). */
 int hsdc_dhssmm(hsdc_ctx *ctx, const double *a, int lda, int m, int n, double *b, int ldb, int k, double tol,
                 int prank, int ni, int ncol, double *time, int *ranks);
